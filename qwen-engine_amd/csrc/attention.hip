@@ -9,6 +9,9 @@
 // [kv_head][max_seq][head_dim] fp16 per layer; q [T][q_dim], k/v [T][kv_dim].
 // Head dim 128: one wave64 covers a head with 2 elements per lane, dot
 // products reduce with DPP/swizzle (seg_sum<64>).
+#include <algorithm>
+#include <type_traits>
+
 #include "attn_common.hpp"
 #include "rope_common.hpp"
 
@@ -400,186 +403,367 @@ __global__ __launch_bounds__(128) void flash_decode_stage2_kernel(const float* _
 }
 
 // ---- causal prefill attention (matrix cores) ---------------------------------------
-// grid (num_q_heads / WPB, ceil(T/32)), WPB waves: wave w is q head
-// blockIdx.x*WPB + w (the WPB heads of a block share one kv head), the block's
-// 32 queries are m0..m0+31 (position base + m; keys [0, base + m]).
-// v_mfma_f32_32x32x16_f16 with queries as the columns:
-//   S^T (32 keys x 32 queries) = K (keys x 128 dims) . Q^T — lane l holds key
-//   row l%32 / query column l%32, dims 8*(l/32) + 16*kk: one 16-byte load each
-//   from the K cache and from q, no LDS;
-//   the result has lane l = query l%32 holding 16 keys (8*(v/4) + 4*(l/32) +
-//   v%4), so a query's max and sum are 16 in-lane values plus one lane^32 swap;
-//   O^T (128 dims x 32 queries) += V^T . P^T — P^T is the lane's own 16
+// The query heads of a kv head and the queries form one list of rows, row
+// r = query r / group, head kvh * group + r % group: a block takes 128
+// consecutive rows (32 per wave) of one kv head, whatever the group size, and
+// its waves share the K and V tiles (64 keys) in LDS.  grid.x = (split, kv
+// head, row block); a split is a run of whole key tiles.  KG = 2: two groups
+// of four waves take alternate tiles of the run and merge through LDS at the end.
+// v_mfma_f32_32x32x16_f16 with the rows as the columns:
+//   S^T (32 keys x 32 rows) = K (keys x 128 dims) . Q^T - lane l holds key
+//   l%32 / row l%32, dims 8*(l/32) + 16*kk; Q stays in registers; the result
+//   has lane l = row l%32 holding 16 keys (8*(v/4) + 4*(l/32) + v%4), so a
+//   row's max and sum are in-lane values plus one lane^32 swap;
+//   O^T (128 dims x 32 rows) += V^T . P^T - P^T is the lane's own
 //   probabilities (fp16, k order = the keys it holds; the k order inside an
-//   MFMA is free when both operands agree) and V^T comes from an LDS tile the
-//   block stores transposed as key pairs (one 32-bit word = two keys of one
-//   dim; rows of 18 words: conflict-free stores and 8-byte reads).
-// Online softmax in the exp2 domain (the 1/sqrt(d) scale folded into the
-// exponent's fused multiply-add), fp32 accumulation; the output is O / L.
-// Tiles wholly below the diagonal and inside the context skip the mask; the
-// accumulator rescale is skipped when no lane's running max moved.
-constexpr int kPqTile = 32;      // queries per block
-constexpr int kPkTile = 32;      // keys per step
-constexpr int kVtWords = 18;     // 32-bit words per LDS row of V^T (16 key pairs + 2 pad)
+//   MFMA is free when both operands agree), V^T comes out of the row-major V
+//   tile through ds_read_b64_tr_b16 (lane i of 16 receives dim i of 4 keys).
+// K and V go from memory straight into LDS (global_load_lds, 16 bytes a lane)
+// a step ahead of their use.  A tile row is 256 bytes, its 16-byte chunk c
+// stored at c ^ swz(key): the 16-byte reads of K (16 keys, one chunk) and the
+// transposing reads of V (4 keys x 4 chunks a half wave) then touch every
+// bank once (0 conflicts counted).
+// Bound by the matrix cores and, beside them, the exponentials: at 1024 rows
+// on 15000 positions (12 q heads, 2 kv heads) 124 us = 790 TFLOP/s, of which the
+// MFMAs alone take 86 us.  Before, every wave read K for itself from L2 and no
+// keys were split: 450 us.  509 rows from position 0 23.2 -> 15.7 us, 4096 rows
+// 211 -> 74 us.
+// Online softmax in the exp2 domain (1/sqrt(d) folded into the exponent's fused
+// multiply-add), fp32 accumulation.  The reference value a row subtracts is
+// its running max, renewed only when the max has grown by more than
+// kPrefillLag (the probabilities then reach at most 2^kPrefillLag, and their
+// relative precision in fp16 does not change); each row decides for itself,
+// so its bits do not depend on the rows beside it.
+constexpr int kPaRows = 128;     // rows per block
+constexpr int kPaKeys = 64;      // keys per tile
+constexpr int kPaTileBytes = kPaKeys * kHeadDim * 2;
+constexpr float kPrefillLag = 8.0f;
+// A split holds at least this many tiles: with 4 instead of 8, 509 rows at
+// position 1000 take 23.0 instead of 23.5 us and 17 rows 13.9 instead of 16.2,
+// 1024 rows from position 0 22.4 instead of 24.3; 2 and 12 are slower (27.8, 23.9).
+constexpr int kPaMinTiles = 4;
+constexpr int kPaMaxSplits = 16;
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-template <int WPB>
-__global__ __launch_bounds__(64 * WPB) void prefill_attention_mfma_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
-    uint16_t* __restrict__ out, const qe_device_control_block* ctl, int T, int nq, int group, int max_seq,
-    int out_stride) {
-    constexpr int NT = 64 * WPB;
-    __shared__ __align__(16) uint32_t sVt[2][kHeadDim * kVtWords];
-    const int qh0 = blockIdx.x * WPB, kvh = qh0 / group, m0 = blockIdx.y * kPqTile;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int qh = qh0 + wave;
+// splits of a row block with `tiles` key tiles, at most `splits`
+__device__ __forceinline__ int prefill_live_splits(int tiles, int splits) {
+    return max(1, min(splits, tiles / kPaMinTiles));
+}
+// key tiles of row block rb (the keys its last row sees)
+__device__ __forceinline__ int prefill_tiles(int rb, int rows, int group, int base, int max_seq) {
+    const int last = min((rb + 1) * kPaRows, rows) - 1;
+    const int len = min(base + last / group + 1, max_seq);
+    return max(0, (len + kPaKeys - 1) / kPaKeys);
+}
+
+struct PrefillAttnParams {
+    const uint16_t* q;
+    const uint16_t* kc;
+    const uint16_t* vc;
+    uint16_t* out;
+    const qe_device_control_block* ctl;
+    float* part_o;   // [split][kv head][row][128] unnormalized
+    float* part_ml;  // [split][kv head][row][2] (reference value, sum)
+    int T, nq, nkv, group, max_seq, out_stride, splits, row_blocks;
+};
+
+__device__ __forceinline__ float xor32_max(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x),
+                                                    false, false);
+    const uint32_t a = r[0], b = r[1];
+    return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+}
+
+// DMA: the caches are 16-byte aligned (else tiles are copied element by element).
+template <int KG, bool DMA>
+__global__ __launch_bounds__(256 * KG, 2) void prefill_attention_kernel(PrefillAttnParams p) {
+    // per key group: K buffers 0 and 1, V buffers 0 and 1
+    __shared__ __align__(16) char smem[KG * 4 * kPaTileBytes];
+    const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int wave = wave_all & 3, kg = wave_all >> 2;
     const int fr = lane & 31, h = lane >> 5;
-    const int base = ctl != nullptr ? ctl->seq_pos : 0;
-    const int m = m0 + fr;                       // this lane's query
-    const int qpos = base + m;                    // its position
-    const int last = min(m0 + kPqTile - 1, T - 1);
-    const int kv_len = min(base + last + 1, max_seq);
-    const int first_diag = base + m0;             // keys below this are visible to every query of the block
-    const size_t hb = static_cast<size_t>(kvh) * max_seq * kHeadDim;
+    const int rb = p.row_blocks - 1 - static_cast<int>(blockIdx.x) % p.row_blocks;  // longest rows first
+    const int cb = static_cast<int>(blockIdx.x) / p.row_blocks;
+    const int kvh = cb % p.nkv, split = cb / p.nkv;
+    const int rows = p.T * p.group;
+    const int base = p.ctl != nullptr ? p.ctl->seq_pos : 0;
+    const int nt_all = prefill_tiles(rb, rows, p.group, base, p.max_seq);
+    const int live = prefill_live_splits(nt_all, p.splits);
+    if (split >= live) return;
+    const int it0 = static_cast<int>((static_cast<long long>(split) * nt_all) / live);
+    const int it1 = static_cast<int>((static_cast<long long>(split + 1) * nt_all) / live);
+    const int r = rb * kPaRows + wave * 32 + fr;
+    const int rc = min(r, rows - 1);
+    const int qi = rc / p.group, qh = kvh * p.group + rc % p.group;
+    const int run_end = it1 * kPaKeys - 1;  // last key of the run
+    const int lim = min(min(base + qi, p.max_seq - 1), run_end);  // last key this row takes here
+    // keys every row of the wave takes: tiles that end at or before it skip the mask
+    const int wave_lim = min(min(base + min(rb * kPaRows + wave * 32, rows - 1) / p.group, p.max_seq - 1), run_end);
+    const int key_max = max(0, min(base + p.T, p.max_seq) - 1);  // the last key that holds anything
     constexpr float kScale = 1.4426950408889634f * 0.08838834764831845f;  // log2(e) / sqrt(128)
 
-    // Q^T operand: 8 k-steps of 16 dims, 8 halves per lane
     u32x4 qf[8];
     {
-        const uint16_t* qr = q + static_cast<size_t>(min(m, T - 1)) * (static_cast<size_t>(nq) * kHeadDim) +
-                             qh * kHeadDim + 8 * h;
+        const uint16_t* qr = p.q + (static_cast<size_t>(qi) * p.nq + qh) * kHeadDim + 8 * h;
 #pragma unroll
         for (int kk = 0; kk < 8; ++kk) qf[kk] = *reinterpret_cast<const u32x4*>(qr + 16 * kk);
     }
+    // tile load i of a wave: tile rows 16 i + 4 wave + lane / 16, stored chunk
+    // lane % 16, i.e. chunk (lane % 16) ^ swz(row) of memory
+    const int lrow = 4 * wave + (lane >> 4);
+    const int lcol = 8 * ((lane & 15) ^ (((lane >> 4) << 2) | wave));
+    const uint32_t loff = static_cast<uint32_t>(2 * (lrow * kHeadDim + lcol));  // bytes
+    const size_t hb = static_cast<size_t>(kvh) * p.max_seq * kHeadDim;
+    const uint16_t* khead = p.kc + hb;
+    const uint16_t* vhead = p.vc + hb;
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+                              (__attribute__((address_space(3))) void*)smem)) + kg * 4 * kPaTileBytes;
+    // Tile t into buffer `buf` (0, 1: K; 2, 3: V).  Written out: the compiler
+    // cannot tell which buffer a load in flight fills and would wait for it at
+    // the next read of LDS; tile_barrier holds the waits.
+    auto load_tile = [&](const uint16_t* head, int t, int buf) __attribute__((always_inline)) {
+        const uint32_t dst = lds0 + buf * kPaTileBytes + wave * 1024;
+        if constexpr (!DMA) {
+            for (int i = 0; i < 4; ++i) {
+                const uint16_t* src = head + static_cast<size_t>(min(t * kPaKeys + 16 * i + lrow, key_max)) * kHeadDim + lcol;
+                uint16_t* to = reinterpret_cast<uint16_t*>(smem + (kg * 4 + buf) * kPaTileBytes + wave * 1024 + 4096 * i + 16 * lane);
+                for (int e = 0; e < 8; ++e) to[e] = src[e];
+            }
+        } else if ((t + 1) * kPaKeys - 1 <= key_max) {  // uniform: one scalar address, one lane offset
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                             ::"s"(dst + 4096 * i), "v"(loff),
+                             "s"(head + (static_cast<size_t>(t) * kPaKeys + 16 * i) * kHeadDim)
+                             : "memory");
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int key = min(t * kPaKeys + 16 * i + lrow, key_max);
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                             ::"s"(dst + 4096 * i), "v"(head + static_cast<size_t>(key) * kHeadDim + lcol)
+                             : "memory");
+            }
+        }
+    };
+    // every tile requested so far is in LDS, for every wave, and what was read before is read
+    auto tile_barrier = [&]() __attribute__((always_inline)) {
+        if constexpr (!DMA) __syncthreads();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // LDS addresses: K chunk 2 kk + h of key fr; V^T reads (dt: 32 dims, u: keys + 8)
+    uint32_t ka[8], va[4][2];
+    {
+        const int swz_k = ((fr & 3) << 2) | ((fr >> 2) & 3);
+        const uint32_t k0 = lds0 + fr * 256 + 16 * (h ^ swz_k);
+        const int s16 = lane & 15, b16 = (lane >> 4) & 1;
+        const uint32_t v0 = lds0 + 2 * kPaTileBytes + (4 * h + (s16 >> 2)) * 256 +
+                            16 * ((2 * b16 + ((s16 & 3) >> 1)) ^ (((s16 >> 2) << 2) | h)) + 8 * (s16 & 1);
+#pragma unroll
+        for (int kk = 0; kk < 8; ++kk) ka[kk] = k0 ^ (32 * kk);
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+            va[dt][0] = v0 ^ (64 * dt);
+            va[dt][1] = (v0 ^ (64 * dt) ^ 32) + 8 * 256;
+        }
+    }
+    // K operand of MFMA i of a tile: 32-key half i % 2, dims 16 (i / 2); V^T
+    // operand: 16-key quarter i / 4, dims 32 (i % 4)
+    auto read_k = [&](int buf, int i) __attribute__((always_inline)) {
+        typedef const __attribute__((address_space(3))) f16x8* lptr;
+        return *reinterpret_cast<lptr>(ka[i >> 1] + buf * kPaTileBytes + (i & 1) * 32 * 256);
+    };
+    auto read_v = [&](int buf, int i) __attribute__((always_inline)) {
+        typedef __attribute__((address_space(3))) s16x4* lptr;
+        const uint32_t off = (buf - 2) * kPaTileBytes + (i >> 2) * 16 * 256;
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lptr>(va[i & 3][0] + off));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lptr>(va[i & 3][1] + off));
+        return __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+
     f32x16 acc[4];
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) acc[dt] = f32x16{};
-    float mrow = -INFINITY, lrow = 0.0f;
-
-    // K and V of a tile are requested two tiles ahead: the loop runs over
-    // pairs of tiles with two register slots (an odd tile count ends with a
-    // fully masked tile), so the loads of tile i + 2 are in flight while tile
-    // i computes and every load is unconditional (positions clamped).
-    constexpr int VC = (kPkTile / 2 * 16 + NT - 1) / NT;  // (key pair, 8 dims) chunks per thread
-    auto load_k = [&](int t0, u32x4 (&kf)[8]) __attribute__((always_inline)) {
-        const int kpos = min(t0 + fr, max_seq - 1);
-        const uint16_t* kr = kc + hb + static_cast<size_t>(kpos) * kHeadDim + 8 * h;
+    float mref = -INFINITY, lsum = 0.0f;
+    auto mask = [&](int t, f32x16 (&sc)[2]) __attribute__((always_inline)) {
+        if ((t + 1) * kPaKeys - 1 > wave_lim) {  // wave-uniform
 #pragma unroll
-        for (int kk = 0; kk < 8; ++kk) kf[kk] = *reinterpret_cast<const u32x4*>(kr + 16 * kk);
-    };
-    // chunk c: key pair c%16 (keys 2(c%16), +1), dims 8*(c/16)..+7
-    auto load_v = [&](int t0, u32x4 (&vr)[VC][2]) __attribute__((always_inline)) {
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int i = 0; i < VC; ++i) {
-            const int c = min(static_cast<int>(threadIdx.x) + NT * i, kPkTile / 2 * 16 - 1);
-            const int kp = c & 15, d0 = 8 * (c >> 4);
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                const int pos = min(t0 + 2 * kp + r, max_seq - 1);
-                vr[i][r] = *reinterpret_cast<const u32x4*>(vc + hb + static_cast<size_t>(pos) * kHeadDim + d0);
-            }
-        }
-    };
-    // -> LDS as V^T key pairs: word (dim d, pair kp) = V[2kp][d] | V[2kp+1][d] << 16
-    auto store_v = [&](const u32x4 (&vr)[VC][2], int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < VC; ++i) {
-            const int c = static_cast<int>(threadIdx.x) + NT * i;
-            if (c < kPkTile / 2 * 16) {
-                const int kp = c & 15, d0 = 8 * (c >> 4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t a = vr[i][0][e], b = vr[i][1][e];  // dims d0+2e (low half), d0+2e+1
-                    sVt[buf][(d0 + 2 * e) * kVtWords + kp] = __builtin_amdgcn_perm(b, a, 0x05040100u);
-                    sVt[buf][(d0 + 2 * e + 1) * kVtWords + kp] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+                for (int v = 0; v < 16; ++v) {
+                    const int key = t * kPaKeys + 32 * j + 8 * (v >> 2) + 4 * h + (v & 3);
+                    sc[j][v] = key <= lim ? sc[j][v] : -INFINITY;
                 }
-            }
         }
     };
-    // one tile: S^T = K . Q^T, online softmax, O^T += V^T . P^T (V^T in sVt[buf])
-    auto tile = [&](int t0, const u32x4 (&kf)[8], int buf) __attribute__((always_inline)) {
-        f32x16 sacc = f32x16{};
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk)
-            sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, kf[kk]),
-                                                          __builtin_bit_cast(f16x8, qf[kk]), sacc, 0, 0, 0);
-        // raw scores of this lane's 16 keys; masked ones -inf
-        float sv[16];
-        if (t0 + kPkTile > first_diag || t0 + kPkTile > kv_len) {  // block-uniform
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int key = t0 + 8 * (v >> 2) + 4 * h + (v & 3);
-                sv[v] = (key < kv_len && key <= qpos && m < T) ? sacc[v] : -INFINITY;
-            }
-        } else {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) sv[v] = sacc[v];
-        }
-        float mx = -INFINITY;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) mx = fmaxf(mx, sv[v]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float mn = fmaxf(mrow, mx * kScale);  // scaling is monotonic: max of the scaled scores
-        const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(mrow - mn);
-        mrow = mn;
-        const float neg = mn == -INFINITY ? 0.0f : -mn;  // masked scores give exp2(-inf) = 0
-        float ps = 0.0f;
-        uint32_t pw[8];
-#pragma unroll
-        for (int v = 0; v < 16; v += 2) {
-            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[v], kScale, neg));
-            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[v + 1], kScale, neg));
-            ps += p0 + p1;
-            pw[v >> 1] = static_cast<uint32_t>(f2h(p0)) | (static_cast<uint32_t>(f2h(p1)) << 16);
-        }
-        lrow = lrow * alpha + ps;
-        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+    auto renew_ref = [&](float mx) __attribute__((always_inline)) {
+        const bool grow = mx > mref + kPrefillLag;
+        if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+            const float alpha = grow ? __builtin_amdgcn_exp2f(mref - mx) : 1.0f;
+            mref = grow ? mx : mref;
+            lsum *= alpha;
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[dt][v] *= alpha;
         }
-        // two 16-key halves of the tile
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const u32x4 pf = {pw[4 * ks], pw[4 * ks + 1], pw[4 * ks + 2], pw[4 * ks + 3]};
-#pragma unroll
-            for (int dt = 0; dt < 4; ++dt) {
-                const uint32_t* row = &sVt[buf][(32 * dt + fr) * kVtWords + 8 * ks + 2 * h];
-                const uint2 lo = *reinterpret_cast<const uint2*>(row);      // keys 16ks + 4h .. +3
-                const uint2 hi = *reinterpret_cast<const uint2*>(row + 4);  // keys 16ks + 8 + 4h .. +3
-                const u32x4 vf = {lo.x, lo.y, hi.x, hi.y};
-                acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, vf),
-                                                                 __builtin_bit_cast(f16x8, pf), acc[dt], 0, 0, 0);
-            }
-        }
     };
-    u32x4 k0[8], k1[8], v0[VC][2], v1[VC][2];
-    load_k(0, k0);
-    load_v(0, v0);
-    load_k(kPkTile, k1);
-    load_v(kPkTile, v1);
-    store_v(v0, 0);
-    __syncthreads();
-    for (int t0 = 0; t0 < kv_len; t0 += 2 * kPkTile) {
-        load_v(t0 + 2 * kPkTile, v0);  // sVt[0] holds tile t0; v0 is free
-        tile(t0, k0, 0);
-        load_k(t0 + 2 * kPkTile, k0);
-        store_v(v1, 1);  // tile t0 + 32, requested one tile ago
-        __syncthreads();
-        load_v(t0 + 3 * kPkTile, v1);
-        tile(t0 + kPkTile, k1, 1);
-        load_k(t0 + 3 * kPkTile, k1);
-        store_v(v0, 0);  // tile t0 + 64
-        __syncthreads();
-    }
-    lrow += __shfl_xor(lrow, 32);
-    if (m < T) {
-        const float inv = lrow > 0.0f ? 1.0f / lrow : 0.0f;
-        uint16_t* o = out + static_cast<size_t>(m) * out_stride + qh * kHeadDim;
+    auto row_max = [&](const f32x16 (&sc)[2]) __attribute__((always_inline)) {
+        float mx = -INFINITY;
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) mx = fmaxf(mx, sc[j][v]);
+        return xor32_max(mx) * kScale;  // scaling is monotonic
+    };
+    // probabilities 2 i and 2 i + 1 of a tile's scores (32-key half i / 8), packed
+    auto probs = [&](const f32x16 (&sc)[2], int i, float neg, float (&ps)[2]) __attribute__((always_inline)) {
+        const int j = i >> 3, v = 2 * (i & 7);
+        const f32x2 e = {__builtin_amdgcn_exp2f(__builtin_fmaf(sc[j][v], kScale, neg)),
+                         __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j][v + 1], kScale, neg))};
+        ps[0] += e.x;
+        ps[1] += e.y;
+        uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(e, f16x2));
+        asm volatile("" : "+v"(w), "+v"(ps[0]), "+v"(ps[1]));  // here, not past the mask's branch
+        return w;
+    };
+    constexpr int AHEAD = 4;  // operand reads in flight before their MFMA
+    // Scores of the K tile in `buf`; beside them, when EXP, the probabilities of
+    // the scores `cur`.  Each MFMA is fenced together with its share of the
+    // vector work: left alone, the scheduler puts all of the one before all
+    // of the other.
+    auto scores = [&](auto exp_too, int buf, f32x16 (&sc)[2], const f32x16 (&cur)[2],
+                      uint32_t (&pw)[2][8]) __attribute__((always_inline)) {
+        const float neg = mref == -INFINITY ? 0.0f : -mref;  // masked scores give exp2(-inf) = 0
+        float ps[2] = {0.0f, 0.0f};
+        f16x8 kf[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) kf[i] = read_k(buf, i);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            sc[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[i % AHEAD], __builtin_bit_cast(f16x8, qf[i >> 1]),
+                                                               i < 2 ? f32x16{} : sc[i & 1], 0, 0, 0);
+            if (i + AHEAD < 16) kf[i % AHEAD] = read_k(buf, i + AHEAD);
+            if constexpr (decltype(exp_too)::value) pw[i >> 3][i & 7] = probs(cur, i, neg, ps);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (decltype(exp_too)::value) lsum += ps[0] + ps[1];
+    };
+    // O^T += V^T . P^T; beside it, when MAX, the (scaled) row maximum of nxt
+    auto add_pv = [&](auto max_too, const uint32_t (&pw)[2][8], int buf, const f32x16 (&nxt)[2]) __attribute__((always_inline)) {
+        f16x8 vf[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) vf[i] = read_v(buf, i);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int j = i >> 3, ks = (i >> 2) & 1, dt = i & 3;
+            const u32x4 pf = {pw[j][4 * ks], pw[j][4 * ks + 1], pw[j][4 * ks + 2], pw[j][4 * ks + 3]};
+            acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i % AHEAD], __builtin_bit_cast(f16x8, pf), acc[dt], 0, 0, 0);
+            if (i + AHEAD < 16) vf[i % AHEAD] = read_v(buf, i + AHEAD);
+            if constexpr (decltype(max_too)::value)
+                mx = fmaxf(fmaxf(mx, nxt[j][2 * (i & 7)]), nxt[j][2 * (i & 7) + 1]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        return decltype(max_too)::value ? xor32_max(mx) * kScale : 0.0f;
+    };
+    typedef std::true_type yes;
+    typedef std::false_type no;
+    // Tile t of the run's scores are in cur: the scores of the group's next tile
+    // beside the probabilities of t, then V of t beside the next tile's maximum.
+    // b: parity of the tile; K of the tile after next and V of the next are requested.
+    auto step = [&](int t, int b, f32x16 (&cur)[2], f32x16 (&nxt)[2]) __attribute__((always_inline)) {
+        uint32_t pw[2][8];
+        load_tile(vhead, t + KG, 2 + (b ^ 1));
+        load_tile(khead, t + 2 * KG, b);
+        scores(yes{}, b ^ 1, nxt, cur, pw);
+        mask(t + KG, nxt);
+        const float mx = add_pv(yes{}, pw, 2 + b, nxt);
+        renew_ref(mx);
+        tile_barrier();
+    };
+    auto finish = [&](int b, f32x16 (&cur)[2]) __attribute__((always_inline)) {
+        uint32_t pw[2][8];
+        const float neg = mref == -INFINITY ? 0.0f : -mref;
+        float ps[2] = {0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 16; ++i) pw[i >> 3][i & 7] = probs(cur, i, neg, ps);
+        lsum += ps[0] + ps[1];
+        add_pv(no{}, pw, 2 + b, cur);
+    };
+    if (it0 < it1) {
+        const int n = (it1 - it0 + KG - 1) / KG;  // tiles of each group; past the run's end every key is masked
+        int t = it0 + kg;
+        load_tile(khead, t, 0);
+        load_tile(vhead, t, 2);
+        load_tile(khead, t + KG, 1);
+        tile_barrier();
+        f32x16 s0[2], s1[2];
+        {
+            uint32_t pw[2][8];
+            scores(no{}, 0, s0, s1, pw);
+        }
+        mask(t, s0);
+        renew_ref(row_max(s0));
+        tile_barrier();  // K buffer 0 is read
+        int left = n;
+        for (; left > 2; left -= 2) {
+            step(t, 0, s0, s1);
+            step(t + KG, 1, s1, s0);
+            t += 2 * KG;
+        }
+        if (left == 2) {
+            step(t, 0, s0, s1);
+            finish(1, s1);
+        } else {
+            finish(0, s0);
+        }
+    }
+    lsum += __shfl_xor(lsum, 32);
+    if constexpr (KG == 2) {
+        // The groups merge: each rescales to the common reference value, hands
+        // over half of its accumulators through the (now idle) tile buffers
+        // and finishes the other half: group 0 dims 0..63, group 1 dims 64..127.
+        float* xch = reinterpret_cast<float*>(smem);  // [group][value][256 threads]
+        float* xml = xch + 2 * 32 * 256;              // [group][2][256 threads]
+        const int gt = wave * 64 + lane;
+        __syncthreads();
+        xml[(kg * 2 + 0) * 256 + gt] = mref;
+        xml[(kg * 2 + 1) * 256 + gt] = lsum;
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) xch[(kg * 32 + d * 16 + v) * 256 + gt] = kg == 0 ? acc[2 + d][v] : acc[d][v];
+        __syncthreads();
+        const float mo = xml[((kg ^ 1) * 2 + 0) * 256 + gt], lo = xml[((kg ^ 1) * 2 + 1) * 256 + gt];
+        const float m = fmaxf(mref, mo);
+        const float wm = mref == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mref - m);
+        const float wo = mo == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mo - m);
+        mref = m;
+        // one order for both groups, so that both hold the same sum
+        const float l0 = kg == 0 ? lsum * wm : lo * wo, l1 = kg == 0 ? lo * wo : lsum * wm;
+        lsum = l0 + l1;
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float mine = kg == 0 ? acc[d][v] : acc[2 + d][v];
+                acc[d][v] = mine * wm + xch[((kg ^ 1) * 32 + d * 16 + v) * 256 + gt] * wo;
+            }
+    }
+    if (r >= rows) return;
+    constexpr int ND = KG == 2 ? 2 : 4;  // 32-dim tiles this wave writes, from dim 64 kg
+    if (live == 1) {
+        const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
+        uint16_t* o = p.out + static_cast<size_t>(qi) * p.out_stride + qh * kHeadDim + 64 * kg;
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {  // dims 32dt + 8g + 4h .. +3
                 const uint32_t w0 = static_cast<uint32_t>(f2h(acc[dt][4 * g] * inv)) |
@@ -588,6 +772,51 @@ __global__ __launch_bounds__(64 * WPB) void prefill_attention_mfma_kernel(
                                     (static_cast<uint32_t>(f2h(acc[dt][4 * g + 3] * inv)) << 16);
                 *reinterpret_cast<uint2*>(o + 32 * dt + 8 * g + 4 * h) = make_uint2(w0, w1);
             }
+        return;
+    }
+    const size_t prow = (static_cast<size_t>(split) * p.nkv + kvh) * rows + r;
+    if (h == 0 && kg == 0) *reinterpret_cast<float2*>(p.part_ml + 2 * prow) = make_float2(mref, lsum);
+    float* po = p.part_o + prow * kHeadDim + 64 * kg;
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<float4*>(po + 32 * dt + 8 * g + 4 * h) =
+                make_float4(acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]);
+}
+
+// Merges the splits of every row: 32 lanes a row (4 dims each), 8 rows a
+// block and pass.  Rows whose block of 128 had one split are already written.
+__global__ __launch_bounds__(256) void prefill_attention_combine_kernel(PrefillAttnParams p) {
+    const int rows = p.T * p.group;
+    const int d = 4 * (threadIdx.x & 31);
+    const int base = p.ctl != nullptr ? p.ctl->seq_pos : 0;
+    const int all = rows * p.nkv;
+    for (int i = blockIdx.x * 8 + (threadIdx.x >> 5); i < all; i += gridDim.x * 8) {
+        const int kvh = i / rows, r = i - kvh * rows;
+        const int live = prefill_live_splits(prefill_tiles(r / kPaRows, rows, p.group, base, p.max_seq), p.splits);
+        if (live == 1) continue;
+        float m = -INFINITY;
+        for (int s = 0; s < live; ++s) m = fmaxf(m, p.part_ml[2 * (static_cast<size_t>(s) * all + i)]);
+        float l = 0.0f;
+        float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        for (int s = 0; s < live; ++s) {
+            const size_t row = static_cast<size_t>(s) * all + i;
+            const float2 ml = *reinterpret_cast<const float2*>(p.part_ml + 2 * row);
+            const float w = ml.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml.x - m);
+            const float4 v = *reinterpret_cast<const float4*>(p.part_o + row * kHeadDim + d);
+            l += w * ml.y;
+            o.x += w * v.x;
+            o.y += w * v.y;
+            o.z += w * v.z;
+            o.w += w * v.w;
+        }
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        uint16_t* dst =
+            p.out + static_cast<size_t>(r / p.group) * p.out_stride + (kvh * p.group + r % p.group) * kHeadDim + d;
+        *reinterpret_cast<uint2*>(dst) =
+            make_uint2(static_cast<uint32_t>(f2h(o.x * inv)) | (static_cast<uint32_t>(f2h(o.y * inv)) << 16),
+                       static_cast<uint32_t>(f2h(o.z * inv)) | (static_cast<uint32_t>(f2h(o.w * inv)) << 16));
     }
 }
 
@@ -688,11 +917,14 @@ extern "C" int qe_launch_attention_gqa_flash_decode_combine(const float* splitk_
     return check_launch("flash_decode_combine");
 }
 
-extern "C" int qe_launch_attention_gqa_prefill(const uint16_t* q, const uint16_t* layer_k_cache,
-                                               const uint16_t* layer_v_cache, uint16_t* attn_out,
-                                               const qe_device_control_block* d_control, int num_tokens,
-                                               hipStream_t stream, int num_q_heads, int num_kv_heads, int head_dim,
-                                               int max_seq_len, int hidden_size) {
+namespace qe {
+
+// Prefill attention; max_context bounds the positions the rows see (the
+// engine knows it on the host, the public entry point only max_seq_len).
+int launch_prefill_attention(const uint16_t* q, const uint16_t* layer_k_cache, const uint16_t* layer_v_cache,
+                             uint16_t* attn_out, const qe_device_control_block* d_control, int num_tokens,
+                             hipStream_t stream, int num_q_heads, int num_kv_heads, int head_dim, int max_seq_len,
+                             int hidden_size, int max_context) {
     QE_REQUIRE(q && layer_k_cache && layer_v_cache && attn_out, "attention_gqa_prefill: NULL pointer");
     QE_REQUIRE(head_dim == kHeadDim, "attention_gqa_prefill: head_dim=%d (only 128 is built)", head_dim);
     QE_REQUIRE(num_kv_heads > 0 && num_q_heads % num_kv_heads == 0, "attention_gqa_prefill: bad head counts");
@@ -700,18 +932,62 @@ extern "C" int qe_launch_attention_gqa_prefill(const uint16_t* q, const uint16_t
     if (num_tokens <= 0) return QE_OK;
     QE_REQUIRE(aligned(q, 16) && aligned(attn_out, 8) && hidden_size % 4 == 0,
                "attention_gqa_prefill: q must be 16-byte and attn_out 8-byte aligned");
-    const int group = num_q_heads / num_kv_heads;
-    // two q heads per block when the group splits evenly (one wave per SIMD,
-    // group/2 blocks per kv head and query tile), else one
-    const int wpb = group % 2 == 0 ? 2 : 1;
-    const dim3 grid(num_q_heads / wpb, (num_tokens + kPqTile - 1) / kPqTile);
-    if (wpb == 2)
-        prefill_attention_mfma_kernel<2><<<grid, 128, 0, stream>>>(q, layer_k_cache, layer_v_cache, attn_out, d_control,
-                                                                   num_tokens, num_q_heads, group, max_seq_len,
-                                                                   hidden_size);
+    PrefillAttnParams p{};
+    p.q = q;
+    p.kc = layer_k_cache;
+    p.vc = layer_v_cache;
+    p.out = attn_out;
+    p.ctl = d_control;
+    p.T = num_tokens;
+    p.nq = num_q_heads;
+    p.nkv = num_kv_heads;
+    p.group = num_q_heads / num_kv_heads;
+    p.max_seq = max_seq_len;
+    p.out_stride = hidden_size;
+    const long long rows = static_cast<long long>(num_tokens) * p.group;
+    const long long row_blocks = (rows + kPaRows - 1) / kPaRows;
+    const long long blocks = row_blocks * num_kv_heads;
+    QE_REQUIRE(rows <= INT32_MAX - kPaRows && blocks <= INT32_MAX, "attention_gqa_prefill: num_tokens=%d", num_tokens);
+    if (blocks == 0) return QE_OK;  // no q heads
+    p.row_blocks = static_cast<int>(row_blocks);
+    // Key splits as far as the chip has room for their blocks (two per CU),
+    // the stream's workspace for their partials, and the context has tiles;
+    // a row block then takes as many of them as its own tiles are worth.
+    const int cus = cu_count();
+    const StreamWorkspace ws = stream_workspace(stream);
+    const long long part = rows * num_kv_heads * (kHeadDim + 2);  // floats of one split
+    p.splits = 1;
+    // (contexts below 16 tiles: the second launch costs what the splits save)
+    if (ws.ptr != nullptr && max_context >= 16 * kPaKeys)
+        p.splits = static_cast<int>(std::max(1LL, std::min({static_cast<long long>(kPaMaxSplits), 2 * cus / blocks,
+                                                            static_cast<long long>(ws.floats) / part,
+                                                            static_cast<long long>(max_context) / (kPaKeys * kPaMinTiles)})));
+    p.part_o = ws.ptr;
+    p.part_ml = ws.ptr + p.splits * rows * num_kv_heads * kHeadDim;
+    // Two key groups per block (one block per CU) once there is more than one
+    // block per CU: blocks half as long leave a smaller last round (4096 rows
+    // from position 0, 384 blocks: 75 against 88 us).  With fewer blocks a
+    // wave that has its SIMD to itself finishes its tiles sooner (509 rows: 13.7
+    // against 16.3 us).
+    if (!aligned(layer_k_cache, 16) || !aligned(layer_v_cache, 16))
+        prefill_attention_kernel<1, false><<<static_cast<unsigned>(blocks * p.splits), 256, 0, stream>>>(p);
+    else if (blocks > cus)
+        prefill_attention_kernel<2, true><<<static_cast<unsigned>(blocks * p.splits), 512, 0, stream>>>(p);
     else
-        prefill_attention_mfma_kernel<1><<<grid, 64, 0, stream>>>(q, layer_k_cache, layer_v_cache, attn_out, d_control,
-                                                                  num_tokens, num_q_heads, group, max_seq_len,
-                                                                  hidden_size);
+        prefill_attention_kernel<1, true><<<static_cast<unsigned>(blocks * p.splits), 256, 0, stream>>>(p);
+    if (p.splits > 1)
+        prefill_attention_combine_kernel<<<static_cast<unsigned>(std::min((rows * num_kv_heads + 7) / 8, 4LL * cus)), 256,
+                                           0, stream>>>(p);
     return check_launch("attention_gqa_prefill");
+}
+
+}  // namespace qe
+
+extern "C" int qe_launch_attention_gqa_prefill(const uint16_t* q, const uint16_t* layer_k_cache,
+                                               const uint16_t* layer_v_cache, uint16_t* attn_out,
+                                               const qe_device_control_block* d_control, int num_tokens,
+                                               hipStream_t stream, int num_q_heads, int num_kv_heads, int head_dim,
+                                               int max_seq_len, int hidden_size) {
+    return qe::launch_prefill_attention(q, layer_k_cache, layer_v_cache, attn_out, d_control, num_tokens, stream,
+                                        num_q_heads, num_kv_heads, head_dim, max_seq_len, hidden_size, max_seq_len);
 }

@@ -284,9 +284,8 @@ int prefill_chunk(qe_engine* e, int start, int len) {
         QE_TRY(qe_launch_qkv_bias_rope_kv_append(e->dq, e->dk, e->dv, L.q_bias, L.k_bias, L.v_bias, kc, vc, e->ctl,
                                                  len, s, c.num_q_heads, c.num_kv_heads, c.head_dim, c.max_seq_len,
                                                  c.head_dim, c.rope_theta));
-        QE_TRY(qe_launch_attention_gqa_prefill(e->dq, kc, vc, e->attn, e->ctl, len, s, c.num_q_heads,
-                                               c.num_kv_heads, c.head_dim, c.max_seq_len,
-                                               c.num_q_heads * c.head_dim));
+        QE_TRY(launch_prefill_attention(e->dq, kc, vc, e->attn, e->ctl, len, s, c.num_q_heads, c.num_kv_heads,
+                                        c.head_dim, c.max_seq_len, c.num_q_heads * c.head_dim, start + len));
         const int qd = c.num_q_heads * c.head_dim;
         if (e->tiled) {
             QE_TRY(qe_launch_gemm_prefill_w4a16_tiled(L.to.w, L.to.s, e->attn, e->act0, e->act0, len, H, qd, s));

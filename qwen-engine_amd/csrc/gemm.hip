@@ -70,10 +70,7 @@ __device__ __forceinline__ float silu_mul(float g, float u) {
 // share partials.
 constexpr size_t kWsFloats = size_t(8) << 20;  // 32 MiB
 
-struct Workspace {
-    float* ptr = nullptr;
-    size_t floats = 0;
-};
+using Workspace = StreamWorkspace;
 
 // One 32x32 accumulator fragment whose rows start at r0 and whose lane
 // column is col.  D[i][j] of a 32x32 MFMA tile: j = lane%32,
@@ -1055,6 +1052,9 @@ int current_device(const char* what, int* dev) {
 }
 
 }  // namespace
+
+StreamWorkspace stream_workspace(hipStream_t stream) { return gemm_workspace(stream); }
+
 }  // namespace qe
 
 extern "C" int qe_gemm_reserve_workspace(hipStream_t stream) {

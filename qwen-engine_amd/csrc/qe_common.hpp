@@ -31,6 +31,22 @@ int gemv_forced_bt();      // 0 auto, else GEMV block size (256, 512, 1024)
 int gemv_forced_cap();     // 0 auto, else the largest GEMV grid (larger grids loop over row sets)
 int engine_tiled_prefill();  // engines created from now on keep tiled copies for the prefill GEMMs (default 1)
 
+// The split workspace registered for a stream (qe_gemm_reserve_workspace /
+// qe_gemm_attach_workspace), {nullptr, 0} without one.  A launch may use it
+// from its first kernel to its last: later work on the stream waits for it.
+struct StreamWorkspace {
+    float* ptr = nullptr;
+    size_t floats = 0;
+};
+StreamWorkspace stream_workspace(hipStream_t stream);
+
+// qe_launch_attention_gqa_prefill for callers that know a bound on the context
+// length the rows see (attention.hip).
+int launch_prefill_attention(const uint16_t* q, const uint16_t* layer_k_cache, const uint16_t* layer_v_cache,
+                             uint16_t* attn_out, const qe_device_control_block* d_control, int num_tokens,
+                             hipStream_t stream, int num_q_heads, int num_kv_heads, int head_dim, int max_seq_len,
+                             int hidden_size, int max_context);
+
 inline int fail(int code, const char* fmt, ...) {
     char buf[512];
     va_list ap;

@@ -303,6 +303,48 @@ def test_engine_prefill_lm_head_matches_oracle(qe, orc):
         e.close()
 
 
+@pytest.mark.parametrize("shift", [0, 1])  # caches 16-byte aligned, or one element off
+@pytest.mark.parametrize("T,base,nq,nkv,max_seq,ws", [
+    (21, 0, 12, 2, 512, True), (22, 511, 12, 2, 4096, True), (64, 448, 12, 2, 2048, True), (509, 0, 12, 2, 4096, True),
+    (43, 1500, 12, 2, 4096, True), (43, 1500, 12, 2, 4096, False), (300, 1800, 8, 8, 2100, True),
+    (5, 2043, 7, 1, 2048, True), (30, 2030, 12, 2, 2048, True), (1100, 0, 32, 32, 1100, True),
+    (1100, 60, 32, 32, 1200, False), (2, 300, 64, 1, 512, True)])
+def test_prefill_attention_splits_and_groups(qe, T, base, nq, nkv, max_seq, ws, shift):
+    """Row blocks, key splits (with and without a stream workspace) and the two
+    key groups (more than one block per CU) against float64; the cache past the
+    context holds NaN and must not be used.  Bound: fp16 output rounding 2^-11
+    and fp16 probabilities (relative 2^-11 each, sum of squares of weights <= 1)
+    against the largest |v| of about 4.5: 4.5 * 2^-10 + 2^-11."""
+    D = 128
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T * 7 + base)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g).half()
+    cache = lambda: rnd(nkv * max_seq * D + 8)[shift:shift + nkv * max_seq * D].view(nkv, max_seq, D)
+    q, kc, vc = rnd(T, nq * D), cache(), cache()
+    end = min(base + T, max_seq)
+    kc[:, end:] = float("nan")
+    vc[:, end:] = float("nan")
+    out = empty((T, nq * D), torch.float16)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    if ws:
+        qe.gemm_reserve_workspace(s)
+    qe.launch_attention_gqa_prefill(q, kc, vc, out, _ctl(base), T, stream=s, num_q_heads=nq, num_kv_heads=nkv,
+                                    head_dim=D, max_seq_len=max_seq, hidden_size=nq * D)
+    s.synchronize()
+    if ws:
+        qe.gemm_release_workspace(s)
+    got = out.double().reshape(T, nq, D)
+    assert torch.isfinite(got).all()
+    pos = torch.arange(base, base + T, device="cuda").clamp(max=max_seq - 1)
+    key = torch.arange(end, device="cuda")
+    for h in range(nq):
+        k, v = kc[h // (nq // nkv), :end].double(), vc[h // (nq // nkv), :end].double()
+        sc = (q.reshape(T, nq, D)[:, h].double() @ k.T) / math.sqrt(D)
+        ref = torch.softmax(sc.masked_fill(key[None] > pos[:, None], -math.inf), -1) @ v
+        assert (got[:, h] - ref).abs().max().item() <= 4.5 * 2.0 ** -10 + 2.0 ** -11
+
+
 def test_engine_tiled_prefill_matches_qwenbin_layout(qe):
     """The engine's prefill on the tiled weight copies gives the same hidden
     rows, logits and tokens as on the .qwenbin layout for the same GEMM plan,
