@@ -105,11 +105,10 @@ __global__ __launch_bounds__(256) void qkv_bias_rope_kv_append_kernel(
 }
 
 // ---- flash decode, stage 1 -----------------------------------------------------
-// grid (num_q_heads, kSplits), NT = 512 threads, one q head per block (GH = 1:
+// grid num_q_heads * kSplits, NT = 512 threads, one q head per block (GH = 1:
 // the group's blocks each re-read the kv head's K and V rows, from L2 after
-// the first, and every block merges one head's lane-group states; measured
-// against half a GQA group per block: 2.85 vs 3.83 us at 128 positions, 4.27
-// vs 6.52 us at 3000, the same bits per head).  A split is a contiguous run of
+// the first, and every block merges one head's lane-group states; half a GQA
+// group per block measured slower, the same bits per head).  A split is a contiguous run of
 // flash_split_len(seq_len) positions (the reference's ceil(seq_len / 16), at
 // least kFlashMinSplit).  The NT/16 lane groups of the block (16 lanes each)
 // each take one position per step; lane j of a group holds dims 8j..8j+7 (one
@@ -192,9 +191,16 @@ __device__ __forceinline__ void flash_round(FlashState<GH>& S, const u32x4 (&qra
     }
 }
 
+// 16 bytes of a cache row that other blocks on the XCD read too (SHARED), or that nobody reads again.
+template <bool SHARED>
+__device__ __forceinline__ u32x4 load_row(const uint16_t* p) {
+    if constexpr (SHARED) return *reinterpret_cast<const u32x4*>(p);
+    return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+}
+
 // One block: GH q heads (qh0..qh0+GH-1) of kv head kvh over positions [t0, t1)
 // with NT threads (NT/16 lane groups).
-template <int GH, int NT>
+template <int GH, int NT, bool SHARED>
 __device__ __forceinline__ void flash_decode_split(const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
                                                    float* __restrict__ part_o, float* __restrict__ part_lse,
                                                    const u32x4 (&qraw)[GH], u32x4 (&ka)[64 / (NT / 16)],
@@ -203,15 +209,6 @@ __device__ __forceinline__ void flash_decode_split(const uint16_t* __restrict__ 
     constexpr int NG = NT / 16, kSteps = 64 / NG;
     const int gid = threadIdx.x >> 4, j = threadIdx.x & 15;  // lane group of the block, lane in the group
     const size_t base = static_cast<size_t>(kvh) * max_seq * kHeadDim + 8 * j;
-    // every load is unconditional (positions clamped to the split)
-    auto load_round = [&](int r0, u32x4 (&kr)[kSteps], u32x4 (&vr)[kSteps]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int st = 0; st < kSteps; ++st) {
-            const int t = min(r0 + st * NG + gid, t1 - 1);
-            kr[st] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kc + base + static_cast<size_t>(t) * kHeadDim));
-            vr[st] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vc + base + static_cast<size_t>(t) * kHeadDim));
-        }
-    };
     FlashState<GH> S;
 #pragma unroll
     for (int h = 0; h < GH; ++h) {
@@ -220,10 +217,24 @@ __device__ __forceinline__ void flash_decode_split(const uint16_t* __restrict__ 
 #pragma unroll
         for (int i = 0; i < 8; ++i) S.o[h][i] = 0.0f;
     }
-    if (t1 - t0 <= 64) {  // one round (every split of a context up to 16 * 64 positions)
+    if (t0 == split * kFlashMinSplit && t1 - t0 <= 64) {  // the rows requested ahead (contexts up to 16 * 64 positions)
         flash_round<GH, NG>(S, qraw, ka, va, t0, t1, gid);
-    } else {  // ping-pong: the next round's rows are in flight while this one is used
+    } else {
+        // rounds of 64 positions in two register slots: the next round's rows
+        // are in flight while this one is used (rounds of 128 and 256 positions
+        // measure the same or slower).  Every load is unconditional (positions
+        // clamped to the split); cached when other q heads of the group read
+        // the same rows through the same L2, else not kept.
+        auto load_round = [&](int r0, u32x4 (&kr)[kSteps], u32x4 (&vr)[kSteps]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int st = 0; st < kSteps; ++st) {
+                const size_t off = base + static_cast<size_t>(min(r0 + st * NG + gid, t1 - 1)) * kHeadDim;
+                kr[st] = load_row<SHARED>(kc + off);
+                vr[st] = load_row<SHARED>(vc + off);
+            }
+        };
         u32x4 kb[kSteps], vb[kSteps];
+        load_round(t0, ka, va);
         for (int r0 = t0;;) {
             load_round(min(r0 + 64, t1 - 1), kb, vb);
             __builtin_amdgcn_sched_barrier(0);
@@ -305,9 +316,8 @@ __device__ __forceinline__ void flash_decode_split(const uint16_t* __restrict__ 
     }
 }
 
-// grid (num_kv_heads * group / GH, kSplits): block x covers q heads
-// GH*x .. GH*x + GH - 1 (kv head GH*x / group).
-template <int GH, int NT>
+// grid num_kv_heads * group / GH * kSplits: a block covers GH q heads of one kv head and split.
+template <int GH, int NT, bool SHARED>
 __global__ __launch_bounds__(NT) void flash_decode_stage1_kernel(const uint16_t* __restrict__ q,
                                                                  const uint16_t* __restrict__ kc,
                                                                  const uint16_t* __restrict__ vc,
@@ -316,8 +326,17 @@ __global__ __launch_bounds__(NT) void flash_decode_stage1_kernel(const uint16_t*
                                                                  const qe_device_control_block* ctl, int group,
                                                                  int max_seq) {
     constexpr int NG = NT / 16, kSteps = 64 / NG;
-    const int qh0 = blockIdx.x * GH, split = blockIdx.y;
-    const int kvh = qh0 / group;
+    // The blocks of a kv head's split (its group's q heads) share an L2: block b
+    // runs on XCD b % 8 (workgroups are dealt out round robin), so unit u =
+    // (split, kv head) takes blocks with b % 8 = u % 8.  With heads in launch
+    // order every XCD fetched every row: 3.43 -> 2.69 us at 128 positions, 7.1
+    // -> 4.4 at 3000, 19.4 -> 10.4 at 16000 (12 q heads, 2 kv heads).
+    static_assert(kSplits % 8 == 0, "units fill the XCDs evenly");
+    const int heads = group / GH;  // blocks per unit
+    const int x = blockIdx.x & 7, sl = blockIdx.x >> 3;
+    const int unit = x + 8 * (sl / heads);
+    const int split = unit % kSplits, kvh = unit / kSplits;
+    const int qh0 = kvh * group + (sl % heads) * GH;
     const int gid = threadIdx.x >> 4, j = threadIdx.x & 15;
     // q and the split's first 64 rows are requested before the position is
     // known: with splits of 64 positions (contexts up to 16 * 64) the rows are
@@ -330,9 +349,9 @@ __global__ __launch_bounds__(NT) void flash_decode_stage1_kernel(const uint16_t*
         const size_t base = static_cast<size_t>(kvh) * max_seq * kHeadDim + 8 * j;
 #pragma unroll
         for (int st = 0; st < kSteps; ++st) {
-            const int t = min(split * kFlashMinSplit + st * NG + gid, max_seq - 1);
-            ka[st] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kc + base + static_cast<size_t>(t) * kHeadDim));
-            va[st] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vc + base + static_cast<size_t>(t) * kHeadDim));
+            const size_t off = base + static_cast<size_t>(min(split * kFlashMinSplit + st * NG + gid, max_seq - 1)) * kHeadDim;
+            ka[st] = load_row<SHARED>(kc + off);
+            va[st] = load_row<SHARED>(vc + off);
         }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -349,16 +368,7 @@ __global__ __launch_bounds__(NT) void flash_decode_stage1_kernel(const uint16_t*
         }
         return;
     }
-    if (per != kFlashMinSplit) {  // longer splits: the first round starts elsewhere
-        const size_t base = static_cast<size_t>(kvh) * max_seq * kHeadDim + 8 * j;
-#pragma unroll
-        for (int st = 0; st < kSteps; ++st) {
-            const int t = min(t0 + st * NG + gid, t1 - 1);
-            ka[st] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kc + base + static_cast<size_t>(t) * kHeadDim));
-            va[st] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vc + base + static_cast<size_t>(t) * kHeadDim));
-        }
-    }
-    flash_decode_split<GH, NT>(kc, vc, part_o, part_lse, qraw, ka, va, kvh, qh0, split, t0, t1, max_seq);
+    flash_decode_split<GH, NT, SHARED>(kc, vc, part_o, part_lse, qraw, ka, va, kvh, qh0, split, t0, t1, max_seq);
 }
 
 // ---- flash decode, stage 2 + Q8_1 epilogue ---------------------------------------
@@ -869,9 +879,13 @@ int launch_flash_stage1(const uint16_t* q, const uint16_t* kc, const uint16_t* v
                num_q_heads, num_kv_heads);
     const int group = num_q_heads / num_kv_heads;
     QE_REQUIRE(max_seq_len > 0, "%s: max_seq_len=%d", what, max_seq_len);
-    const dim3 grid(num_q_heads, kSplits);
-    flash_decode_stage1_kernel<1, kFlashThreads><<<grid, kFlashThreads, 0, stream>>>(q, kc, vc, part_o, part_lse, ctl,
-                                                                                    group, max_seq_len);
+    static_assert(kSplits % 8 == 0, "units fill the XCDs evenly");
+    if (group > 1)
+        flash_decode_stage1_kernel<1, kFlashThreads, true><<<num_q_heads * kSplits, kFlashThreads, 0, stream>>>(
+            q, kc, vc, part_o, part_lse, ctl, group, max_seq_len);
+    else
+        flash_decode_stage1_kernel<1, kFlashThreads, false><<<num_q_heads * kSplits, kFlashThreads, 0, stream>>>(
+            q, kc, vc, part_o, part_lse, ctl, group, max_seq_len);
     return QE_OK;
 }
 }  // namespace
