@@ -26,153 +26,13 @@
 #include <atomic>
 #include <mutex>
 
-#include "qe_common.hpp"
+#include "gemm_common.hpp"
 
 
 namespace qe {
 namespace {
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kPlain = 0;
-constexpr int kQKV = 1;
-constexpr int kSwiglu = 2;
-constexpr int BK = 64;
 constexpr int A_STRIDE = 72;  // halves per LDS row of the A tile (64 + 8 pad)
-
-struct GemmParams {
-    const uint32_t* qw[3];
-    const uint16_t* sc[3];
-    uint16_t* out[3];
-    int col_begin[3];  // first virtual column of each matrix (QKV)
-    int out_stride[3]; // row stride of each output
-    const uint16_t* A;
-    const uint16_t* residual;
-    const int8_t* A8;         // W4A8 variant: Q8_1 rows of the activation
-    const float* A8_scale;
-    const int32_t* A8_sum8;
-    float* ws;         // split-K partials (slices > 1 only)
-    int M, N, K;       // N = virtual columns (SwiGLU: 2*I)
-};
-
-// silu(g) * u = g * u / (1 + e^-g) with the hardware exp2 and reciprocal
-// (about 1 ulp each in fp32; the result is rounded to fp16)
-__device__ __forceinline__ float silu_mul(float g, float u) {
-    return g * u * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * g));
-}
-
-// Split-K partials: fp32 tiles of the K slices, reduced by a second kernel
-// on the same stream (deterministic order, no atomics or fences).  They live
-// in a workspace of kWsFloats floats that belongs to the launching stream
-// (gemm_workspace below), so GEMMs in flight on different streams never
-// share partials.
-constexpr size_t kWsFloats = size_t(8) << 20;  // 32 MiB
-
-using Workspace = StreamWorkspace;
-
-// One 32x32 accumulator fragment whose rows start at r0 and whose lane
-// column is col.  D[i][j] of a 32x32 MFMA tile: j = lane%32,
-// i = 8*(v/4) + 4*(lane/32) + v%4
-// Value of the neighbouring lane (lane ^ 1), by DPP within the quad.
-__device__ __forceinline__ float swap_adjacent(float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, false));
-}
-
-template <int MODE>
-__device__ __forceinline__ void epilogue_frag(const GemmParams& p, const f32x16& acc, int r0, int col, int lane) {
-    const int fr = lane & 31;
-    // rows of element v: r0 + 8 * (v / 4) + 4 * (lane / 32) + v % 4 (static
-    // offsets from the lane's first row; every index into acc is static)
-    const int lrow = r0 + 4 * (lane >> 5);
-    const bool cols_ok = col < p.N;
-    const bool rows_ok = r0 + 32 <= p.M;  // the whole fragment: no per-row checks
-    if constexpr (MODE == kSwiglu) {
-        // lane pair (gate column, up column): the gate lane finishes rows
-        // v < 8 and the up lane rows v >= 8 (16 further down), so every lane
-        // evaluates 8 silu; the partner's values arrive by DPP swaps
-        const bool gate = (fr & 1) == 0;
-        const int row0 = lrow + (gate ? 0 : 16);
-        const int stride = p.out_stride[0];
-        uint16_t* out = p.out[0] + (col >> 1);
-#pragma unroll
-        for (int v = 0; v < 8; ++v) {
-            const float lo = acc[v], hi = acc[v + 8];
-            const float lo_x = swap_adjacent(lo), hi_x = swap_adjacent(hi);
-            const float g = gate ? lo : hi_x;
-            const float u = gate ? lo_x : hi;
-            const int row = row0 + 8 * (v >> 2) + (v & 3);
-            if (cols_ok && (rows_ok || row < p.M)) out[static_cast<size_t>(row) * stride] = f2h(silu_mul(g, u));
-        }
-        return;
-    }
-    int m = 0, local = col;
-    if constexpr (MODE == kQKV) {
-        m = (col >= p.col_begin[1]) + (col >= p.col_begin[2]);
-        local = col - p.col_begin[m];
-    }
-    const int stride = MODE == kQKV ? (m == 0 ? p.out_stride[0] : m == 1 ? p.out_stride[1] : p.out_stride[2])
-                                    : p.out_stride[0];
-    uint16_t* out = (MODE == kQKV ? (m == 0 ? p.out[0] : m == 1 ? p.out[1] : p.out[2]) : p.out[0]) + local;
-    const uint16_t* res = (MODE == kPlain && p.residual != nullptr) ? p.residual + local : nullptr;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int row = lrow + 8 * (v >> 2) + (v & 3);
-        if (cols_ok && (rows_ok || row < p.M)) {
-            const size_t off = static_cast<size_t>(row) * stride;
-            _Float16 h = static_cast<_Float16>(acc[v]);
-            if (MODE == kPlain && res != nullptr) h = h + __builtin_bit_cast(_Float16, res[off]);  // fp16 add, RNE
-            out[off] = __builtin_bit_cast(uint16_t, h);
-        }
-    }
-}
-
-template <int BM, int BN, int WGM, int MODE>
-__device__ __forceinline__ void epilogue(const GemmParams& p, const f32x16 (&acc)[BM / WGM / 32][BN / (4 / WGM) / 32],
-                                         int m0, int n0, int wm, int wn, int lane) {
-    constexpr int WM = BM / WGM, WN = BN / (4 / WGM), MI = WM / 32, NI = WN / 32;
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j)
-            epilogue_frag<MODE>(p, acc[i][j], m0 + wm * WM + i * 32, n0 + wn * WN + j * 32 + (lane & 31), lane);
-}
-
-// Nibble order of a word of the tiled copy: k0 at bits 0-3, k1 at 16-19, k2 at
-// 4-7, k3 at 20-23, k4 at 8-11, k5 at 24-27, k6 at 12-15, k7 at 28-31.  A
-// nibble in bits 0-3 of a 16-bit half under the exponent of 1024.0 (0x6400)
-// reads as 1024 + q; in bits 4-7 under the exponent of 64.0 (0x5400) as
-// 64 + q.  So the 8 values in K order cost five bit operations (two masked
-// ORs, a shift, two masked ORs), then the exact subtraction of 1032 or 72 and
-// the one fp16 RNE multiply by the scale of unpack_w4_to_half8 - the same
-// values as unpack_w4_to_half8 on the original word.
-// The four masks live in VGPRs (TiledMasks, set up once per kernel): gfx9
-// VOP3 instructions take no literal constants, so with literal masks the
-// compiler emits separate AND and OR instructions instead of V_AND_OR_B32.
-struct TiledMasks {
-    uint32_t lo, hi, bias_lo, bias_hi;
-};
-__device__ __forceinline__ TiledMasks tiled_masks() {
-    TiledMasks m{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
-    asm volatile("" : "+v"(m.lo), "+v"(m.hi), "+v"(m.bias_lo), "+v"(m.bias_hi));
-    return m;
-}
-__device__ __forceinline__ qwen::qe_half8_t unpack_w4t_to_half8(uint32_t w, _Float16 scale, const TiledMasks& m) {
-    const uint32_t w8 = w >> 8;
-    const uint32_t u01 = (w & m.lo) | m.bias_lo;
-    const uint32_t u23 = (w & m.hi) | m.bias_hi;
-    const uint32_t u45 = (w8 & m.lo) | m.bias_lo;
-    const uint32_t u67 = (w8 & m.hi) | m.bias_hi;
-    const qwen::qe_half2_t b1 = {(_Float16)1032.0f, (_Float16)1032.0f};
-    const qwen::qe_half2_t b2 = {(_Float16)72.0f, (_Float16)72.0f};
-    const qwen::qe_half2_t sc = {scale, scale};
-    const qwen::qe_half2_t h01 = (__builtin_bit_cast(qwen::qe_half2_t, u01) - b1) * sc;
-    const qwen::qe_half2_t h23 = (__builtin_bit_cast(qwen::qe_half2_t, u23) - b2) * sc;
-    const qwen::qe_half2_t h45 = (__builtin_bit_cast(qwen::qe_half2_t, u45) - b1) * sc;
-    const qwen::qe_half2_t h67 = (__builtin_bit_cast(qwen::qe_half2_t, u67) - b2) * sc;
-    return qwen::qe_half8_t{h01[0], h01[1], h23[0], h23[1], h45[0], h45[1], h67[0], h67[1]};
-}
 
 // The same 8 values of an original word, in the tiled word's nibble order.
 __device__ __forceinline__ uint32_t w4_word_to_tiled(uint32_t w) {
@@ -614,56 +474,6 @@ __global__ __launch_bounds__(512, 1) void gemm_w4a16_ks2_kernel(GemmParams p) {
     }
 }
 
-// Sums the K-slice partials in slice order and applies the epilogue.  grid
-// (N tiles, M tiles, fragments): block z takes the 32x32 fragment z of its
-// tile, 256 threads in the MFMA lane layout of the 4 waves.  S > 0: all S
-// slices are requested before the first add (one memory latency, not S);
-// S = 0: a loop over the slices.
-template <int BM, int BN, int WGM, int MODE, int S>
-__global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmParams p, int slices) {
-    constexpr int WGN = 4 / WGM;
-    constexpr int WM = BM / WGM, WN = BN / WGN, NI = WN / 32;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int tile = blockIdx.y * gridDim.x + blockIdx.x;
-    const int n_tiles = gridDim.x * gridDim.y;
-    const int f = blockIdx.z, i = f / NI, j = f % NI;
-    const size_t slice_stride = static_cast<size_t>(n_tiles) * (BM * BN);
-    const float* part = p.ws + static_cast<size_t>(tile) * (BM * BN) + f * 16 * 256 + tid;
-    f32x16 acc = f32x16{};
-    if constexpr (S > 0) {
-        float x[S][16];
-#pragma unroll
-        for (int z = 0; z < S; ++z)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) x[z][v] = part[z * slice_stride + v * 256];
-#pragma unroll
-        for (int z = 0; z < S; ++z)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[v] += x[z][v];
-    } else {
-        for (int z = 0; z < slices; ++z)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[v] += part[z * slice_stride + v * 256];
-    }
-    const int wm = wave / WGN, wn = wave % WGN;
-    epilogue_frag<MODE>(p, acc, blockIdx.y * BM + wm * WM + i * 32, blockIdx.x * BN + wn * WN + j * 32 + (lane & 31),
-                        lane);
-}
-
-template <int BM, int BN, int WGM, int MODE>
-void launch_reduce(const GemmParams& p, dim3 tiles, int slices, hipStream_t s) {
-    constexpr int FR = (BM / WGM / 32) * (BN / (4 / WGM) / 32);  // fragments per wave
-    const dim3 grid(tiles.x, tiles.y, FR);
-    switch (slices) {
-        case 2: gemm_splitk_reduce_kernel<BM, BN, WGM, MODE, 2><<<grid, 256, 0, s>>>(p, slices); break;
-        case 3: gemm_splitk_reduce_kernel<BM, BN, WGM, MODE, 3><<<grid, 256, 0, s>>>(p, slices); break;
-        case 4: gemm_splitk_reduce_kernel<BM, BN, WGM, MODE, 4><<<grid, 256, 0, s>>>(p, slices); break;
-        case 6: gemm_splitk_reduce_kernel<BM, BN, WGM, MODE, 6><<<grid, 256, 0, s>>>(p, slices); break;
-        case 8: gemm_splitk_reduce_kernel<BM, BN, WGM, MODE, 8><<<grid, 256, 0, s>>>(p, slices); break;
-        default: gemm_splitk_reduce_kernel<BM, BN, WGM, MODE, 0><<<grid, 256, 0, s>>>(p, slices); break;
-    }
-}
-
 template <int BM, int BN, int WGM, int MODE, bool TILED = false>
 void launch_tiles(const GemmParams& p, int slices, hipStream_t s) {
     const dim3 grid((p.N + BN - 1) / BN, (p.M + BM - 1) / BM, slices);
@@ -722,16 +532,57 @@ float predict_us(const TileCost& t, int M, int N, int K, int slices, int cus) {
     return us;
 }
 
+// The tiled-weight kernels with both operands through LDS (gemm_dma.hip), fitted
+// to a sweep of tiles x slices over M in {128..4096} at the Qwen2.5-1.5B shapes
+// (rms error 5 %): fixed cost, cost of a further round of blocks, per-64-k-step
+// cost of a nearly empty and the increase to a full round (one k group: with one
+// block per CU and with two), split-K cost and cost per MB of partials.
+struct DmaCost {
+    int bm, bn, groups;
+    float fixed, round, step1, fill1, step2, fill2, split, split_mb;
+};
+constexpr int kDmaTiles = 3;  // gemm_tile 5, 6, 7
+constexpr DmaCost kDma[kDmaTiles] = {
+    {128, 256, 1, 8.03f, 12.3f, 0.774f, 0.063f, 1.223f, 0.199f, 0.0f, 0.054f},
+    {128, 256, 2, 7.17f, 8.90f, 1.239f, 0.153f, 1.239f, 0.153f, 1.54f, 0.051f},
+    {128, 128, 2, 4.93f, 4.99f, 0.750f, 0.131f, 0.750f, 0.131f, 2.84f, 0.081f},
+};
+
+float predict_dma_us(const DmaCost& t, int M, int N, int K, int slices, int cus) {
+    const long long tiles = static_cast<long long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    const long long blocks = tiles * slices;
+    const long long slots = t.groups == 1 ? 2LL * cus : cus;
+    const int quads = (K / 256 + slices - 1) / slices;
+    const float steps = 4.0f * static_cast<float>((quads + t.groups - 1) / t.groups);
+    const long long rounds = (blocks + slots - 1) / slots, last = blocks - (rounds - 1) * slots;
+    const float u = static_cast<float>(last) / static_cast<float>(slots);
+    float us = t.fixed + (static_cast<float>(rounds - 1) + u) * t.round +
+               static_cast<float>(rounds - 1) * steps * (t.step2 + t.fill2);
+    if (last <= cus) us += steps * (t.step1 + t.fill1 * static_cast<float>(last) / static_cast<float>(cus));
+    else us += steps * (t.step2 + t.fill2 * u);
+    if (slices > 1) us += t.split + t.split_mb * (static_cast<float>(blocks) * t.bm * t.bn * 8.0f / 1e6f);
+    return us;
+}
+
 // Tile and K-slice plan of a prefill GEMM: the configuration the time model
 // predicts fastest among those whose split-K partials fit ws_floats, then the
-// gemm_tile / gemm_slices overrides.
+// gemm_tile / gemm_slices overrides.  ti: 0..3 the register-staged tiles, 4..6
+// the kernels of gemm_dma.hip (tiled weights only).  Those win where a launch
+// has enough steps to fill (gate/up at M = 1024 72 against 78 us, 2048 120
+// against 136, 4096 215 against 265; down at M = 2048 70 against 80; QKV at M =
+// 2048 19.6 against 25) and lose 1 to 6 us on shorter ones (QKV at M = 512 15.7
+// against 10.0).  The register-staged model is 10 % low around the crossing and
+// 15 to 25 % low past M = 1280, hence the factors.
 void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& slices) {
     const int cus = cu_count();
     const int KT = K / BK;
     const int max_slices = (K % 256 == 0) ? KT / 4 : KT;  // QUAD slices whole 256-k quads
-    auto fits = [&](const TileCost& t, int s) {
-        const size_t tiles = static_cast<size_t>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-        return s == 1 || (s <= max_slices && KT / s >= 4 && static_cast<size_t>(s) * tiles * t.bm * t.bn <= ws_floats);
+    auto fits_tile = [&](int bm, int bn, int s) {
+        const size_t tiles = static_cast<size_t>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        return s == 1 || (s <= max_slices && KT / s >= 4 && static_cast<size_t>(s) * tiles * bm * bn <= ws_floats);
+    };
+    auto fits = [&](int i, int s) {
+        return i < 4 ? fits_tile(kTiles[i].bm, kTiles[i].bn, s) : fits_tile(kDma[i - 4].bm, kDma[i - 4].bn, s);
     };
     ti = 0;
     slices = 1;
@@ -739,14 +590,25 @@ void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& 
     for (int i = 0; i < 4; ++i) {
         for (int s : {1, 2, 3, 4, 6}) {
             if (s > 1 && !gemm_split_k_enabled()) break;
-            if (!fits(kTiles[i], s)) continue;
+            if (!fits(i, s)) continue;
             const float us = predict_us(tiled ? kTilesTiled[i] : kTiles[i], M, N, K, s, cus);
             if (us < best) { best = us; ti = i; slices = s; }
         }
     }
-    if (const int f = gemm_forced_tile()) ti = f - 1;
+    if (tiled && M > 64) {
+        best *= M >= 1280 ? 1.25f : 1.12f;
+        for (int i = 4; i < 4 + kDmaTiles; ++i) {
+            for (int s : {1, 2, 3, 4, 6}) {
+                if (s > 1 && !gemm_split_k_enabled()) break;
+                if (!fits(i, s)) continue;
+                const float us = predict_dma_us(kDma[i - 4], M, N, K, s, cus);
+                if (us < best) { best = us; ti = i; slices = s; }
+            }
+        }
+    }
+    if (const int f = gemm_forced_tile(); f >= 1 && (f <= 4 || tiled)) ti = f - 1;
     if (const int f = gemm_forced_slices()) slices = f;
-    while (slices > 1 && !fits(kTiles[ti], slices)) --slices;
+    while (slices > 1 && !fits(ti, slices)) --slices;
 }
 
 template <int MODE>
@@ -756,9 +618,11 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, Workspace ws
     const size_t ws_floats = ws.ptr == nullptr ? 0 : ws.floats;
     int ti = 0, slices = 1;
     plan_gemm(p.M, p.N, p.K, ws_floats, tiled, ti, slices);
-    const TileCost& t = kTiles[ti];
-    if ((p.M + t.bm - 1) / t.bm > 65535) return fail(QE_ERR_UNSUPPORTED, "%s: M=%d too large", what, p.M);
-    if (tiled) {
+    const int bm = ti < 4 ? kTiles[ti].bm : kDma[ti - 4].bm;
+    if ((p.M + bm - 1) / bm > 65535) return fail(QE_ERR_UNSUPPORTED, "%s: M=%d too large", what, p.M);
+    if (ti >= 4) {
+        launch_gemm_dma(MODE, ti - 4, p, slices, stream);
+    } else if (tiled) {
         switch (ti) {
             case 0: launch_tiles<64, 64, 2, MODE, true>(p, slices, stream); break;
             case 1: launch_tiles<64, 128, 1, MODE, true>(p, slices, stream); break;

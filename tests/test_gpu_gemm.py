@@ -444,3 +444,47 @@ def test_gemm_tiled_qkv_and_swiglu_bit_identical(qe, orc):
     assert_fp16_close(host(b)[:8], ex, bd, ref, what="tiled swiglu, own plan")
     with pytest.raises(RuntimeError, match="multiple of 256"):
         qe.launch_gemm_prefill_w4a16_tiled(tw, ts, dev(A), None, b, M, 64, 128)
+
+
+@pytest.mark.parametrize("K", [256, 768, 1280, 2048])  # 1, 3, 5 and 8 quads: uneven k groups and slices
+@pytest.mark.parametrize("tile", [5, 6, 7])
+def test_gemm_tiled_dma_tiles_ragged(qe, orc, tile, K):
+    """The tiled-weight kernels with both operands through LDS, forced, with one,
+    two and three K slices, on rows and columns that end inside a tile and past
+    one: plain with residual, QKV with widths off the column tile, SwiGLU."""
+    from helpers import ulp16
+    M, N, I = 131, 298, 150
+    nq, nkv, hd = 5, 2, 32
+    qw, sc = orc.synth_w4(700 + K, N, K)
+    A = _A(orc, M, K, 14)
+    R = orc.synth_f16_normal(15, M * N).reshape(M, N)
+    dims = (nq * hd, nkv * hd, nkv * hd)
+    mats = [orc.synth_w4(710 + i, n, K) for i, n in enumerate(dims)]
+    gq, gs = orc.synth_w4(720 + K, 2 * I, K)
+    ref_p, ex_p, bd_p = orc.gemm_w4a16(qw, sc, A, M, N, K, residual=R)
+    _, acc_p, _ = orc.gemm_w4a16(qw, sc, A, M, N, K)
+    refs_q = [orc.gemm_w4a16(w, s, A, M, n, K) for (w, s), n in zip(mats, dims)]
+    ref_g, ex_g, bd_g = orc.gemm_swiglu_w4a16(gq, gs, A, M, K, I)
+    dA = dev(A)
+    tw = qe.w4_tiled(dev(qw), dev(sc), N, K)
+    tq = [qe.w4_tiled(dev(w), dev(s), n, K) for (w, s), n in zip(mats, dims)]
+    tg = qe.w4_tiled(dev(gq), dev(gs), 2 * I, K)
+    for slices in (1, 2, 3):
+        what = f"tile {tile} slices {slices} K {K}"
+        print(what, flush=True)
+        with forced_plan(qe, tile, slices):
+            assert qe.gemm_prefill_plan(M, N, K, True) == (tile, min(slices, K // 256))
+            out = dev(R)
+            qe.launch_gemm_prefill_w4a16_tiled(*tw, dA, out, out, M, N, K)
+            outs = [empty((M, n), torch.float16) for n in dims]
+            qe.launch_gemm_prefill_qkv_w4a16_tiled(
+                qe.make_qkv_view(*tq[0], outs[0], *tq[1], outs[1], *tq[2], outs[2]), dA, M, in_features=K,
+                num_q_heads=nq, num_kv_heads=nkv, head_dim=hd)
+            outg = empty((M, I), torch.float16)
+            qe.launch_gemm_prefill_dual_gate_up_swiglu_w4a16_tiled(*tg, dA, outg, M, hidden_size=K,
+                                                                   intermediate_size=I)
+        assert_fp16_close(host(out), ex_p, bd_p + ulp16(acc_p) * 2.0 ** 20, ref_p, what="plain " + what,
+                          max_floor_frac=1.0)  # the floor carries the fp16 rounding of acc
+        for o, (ref, ex, bd) in zip(outs, refs_q):
+            assert_fp16_close(host(o), ex, bd, ref, what="qkv " + what)
+        assert_fp16_close(host(outg), ex_g, bd_g, ref_g, what="swiglu " + what)
