@@ -407,10 +407,11 @@ int qe_stream_read(const void* data, size_t bytes, uint32_t* sink, hipStream_t s
 /* Process-wide tuning switches (no counterpart in the reference):
  *   "gemm_split_k" 0/1 (default 1) - split K across blocks for prefill GEMMs
  *   whose tile grid leaves CUs idle;
- *   "gemm_tile" 0..7 (default 0 = chosen per shape) - force the prefill GEMM
+ *   "gemm_tile" 0..8 (default 0 = chosen per shape) - force the prefill GEMM
  *   block tile: 1 64x64, 2 64x128, 3 128x64, 4 128x128 (rows x columns); tiled
  *   weights only (ignored for others): 5 128x256, 6 128x256 and 7 128x128 with
- *   two k groups a block, both operands through LDS;
+ *   two k groups a block, both operands through LDS; 8 the kernel for up to
+ *   32 rows (ignored for more; never sliced);
  *   "gemm_slices" 0..64 (default 0 = chosen per shape) - force the number of
  *   K slices;
  *   "gemm_ks2" 0..2 (default 0) - prefill GEMMs with K % 256 == 0 split the k

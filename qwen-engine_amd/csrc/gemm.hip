@@ -564,6 +564,18 @@ float predict_dma_us(const DmaCost& t, int M, int N, int K, int slices, int cus)
     return us;
 }
 
+// Time of the kernel for a few rows (gemm_skinny.hip): launch and one load
+// latency, the bytes a block takes from L2 (weights of the .qwenbin layout cost
+// half again, in 64-byte pieces) at 45 GB/s per CU, the weights at 5 TB/s.
+constexpr int kSkinnyTile = 7;  // gemm_tile 8
+float predict_skinny_us(int M, int N, int K, bool tiled, int cus) {
+    const int cols = skinny_columns(M, N);
+    const float wkb = 0.5e-3f * static_cast<float>(K) * (tiled ? 1.0f : 1.5f);  // one column
+    const float blocks = static_cast<float>((N + cols - 1) / cols) / static_cast<float>(cus);
+    const float kb = wkb * static_cast<float>(cols) + 2e-3f * static_cast<float>(M) * static_cast<float>(K);
+    return 3.4f + std::max(1.0f, blocks) * kb * (M > 16 ? 1.4f : 1.0f) / 45.0f + wkb * static_cast<float>(N) / 5e3f;
+}
+
 // Tile and K-slice plan of a prefill GEMM: the configuration the time model
 // predicts fastest among those whose split-K partials fit ws_floats, then the
 // gemm_tile / gemm_slices overrides.  ti: 0..3 the register-staged tiles, 4..6
@@ -606,8 +618,18 @@ void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& 
             }
         }
     }
-    if (const int f = gemm_forced_tile(); f >= 1 && (f <= 4 || tiled)) ti = f - 1;
-    if (const int f = gemm_forced_slices()) slices = f;
+    // a few rows: the tile model is 5 to 15 % high there (gate/up 10.0 against
+    // 10.5 us predicted, down 12.0 against 14.0, tiled)
+    const bool few = M <= kSkinnyRows && gemm_forced_slices() == 0 &&
+                     predict_skinny_us(M, N, K, tiled, cus) < 0.9f * best;
+    if (few) {
+        ti = kSkinnyTile;
+        slices = 1;
+    }
+    const int f = gemm_forced_tile();
+    if ((f >= 1 && f <= 4) || (f >= 5 && f <= 7 && tiled) || (f == kSkinnyTile + 1 && M <= kSkinnyRows)) ti = f - 1;
+    if (const int n = gemm_forced_slices()) slices = n;
+    if (ti == kSkinnyTile) slices = 1;
     while (slices > 1 && !fits(ti, slices)) --slices;
 }
 
@@ -618,6 +640,10 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, Workspace ws
     const size_t ws_floats = ws.ptr == nullptr ? 0 : ws.floats;
     int ti = 0, slices = 1;
     plan_gemm(p.M, p.N, p.K, ws_floats, tiled, ti, slices);
+    if (ti == kSkinnyTile) {
+        launch_gemm_skinny(MODE, p, tiled, stream);
+        return check_launch(what);
+    }
     const int bm = ti < 4 ? kTiles[ti].bm : kDma[ti - 4].bm;
     if ((p.M + bm - 1) / bm > 65535) return fail(QE_ERR_UNSUPPORTED, "%s: M=%d too large", what, p.M);
     if (ti >= 4) {

@@ -207,4 +207,9 @@ void launch_reduce(const GemmParams& p, dim3 tiles, int slices, hipStream_t s) {
 // k groups a block; p.ws holds the partials when slices > 1.
 void launch_gemm_dma(int mode, int tile, const GemmParams& p, int slices, hipStream_t stream);
 
+// The kernel for up to kSkinnyRows rows (gemm_skinny.hip).
+constexpr int kSkinnyRows = 32;
+inline int skinny_columns(int M, int N) { return M <= 16 && N >= 16 * 512 ? 32 : 16; }  // of a block
+void launch_gemm_skinny(int mode, const GemmParams& p, bool tiled, hipStream_t stream);
+
 }  // namespace qe

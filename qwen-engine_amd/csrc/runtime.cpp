@@ -64,7 +64,7 @@ extern "C" int qe_set_tuning(const char* key, int value) {
         return QE_OK;
     }
     if (std::strcmp(key, "gemm_tile") == 0) {
-        if (value < 0 || value > 7) return qe::fail(QE_ERR_INVALID_ARGUMENT, "set_tuning: gemm_tile %d not in 0..7", value);
+        if (value < 0 || value > 8) return qe::fail(QE_ERR_INVALID_ARGUMENT, "set_tuning: gemm_tile %d not in 0..8", value);
         qe::g_gemm_tile = value;
         return QE_OK;
     }

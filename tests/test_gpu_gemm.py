@@ -488,3 +488,50 @@ def test_gemm_tiled_dma_tiles_ragged(qe, orc, tile, K):
         for o, (ref, ex, bd) in zip(outs, refs_q):
             assert_fp16_close(host(o), ex, bd, ref, what="qkv " + what)
         assert_fp16_close(host(outg), ex_g, bd_g, ref_g, what="swiglu " + what)
+
+
+@pytest.mark.parametrize("K", [128, 384, 768, 4096])  # one group, odd groups, whole lines, several rounds a wave
+@pytest.mark.parametrize("M", [1, 16, 17, 32])
+def test_gemm_few_rows(qe, orc, M, K):
+    """The kernel for up to 32 rows, forced, on both layouts: plain with residual
+    (columns that end inside a tile), QKV with head ranges off the column tile,
+    SwiGLU, and a matrix wide enough for 32 columns a block."""
+    from helpers import ulp16
+    N, I, wide = 43, 27, 16 * 512 + 6
+    dims = (120, 40, 40)
+    qw, sc = orc.synth_w4(800 + K, N, K)
+    A = _A(orc, M, K, 16)
+    R = orc.synth_f16_normal(17, M * N).reshape(M, N)
+    mats = [orc.synth_w4(810 + i, n, K) for i, n in enumerate(dims)]
+    gq, gs = orc.synth_w4(820 + K, 2 * I, K)
+    lw, ls = orc.synth_w4(830 + K, wide, K)
+    ref_p, ex_p, bd_p = orc.gemm_w4a16(qw, sc, A, M, N, K, residual=R)
+    _, acc_p, _ = orc.gemm_w4a16(qw, sc, A, M, N, K)
+    refs_q = [orc.gemm_w4a16(w, s, A, M, n, K) for (w, s), n in zip(mats, dims)]
+    ref_g, ex_g, bd_g = orc.gemm_swiglu_w4a16(gq, gs, A, M, K, I)
+    cols = np.r_[0:40, wide - 40:wide]
+    ref_w, ex_w, bd_w = orc.gemm_w4a16(np.ascontiguousarray(lw[cols]), np.ascontiguousarray(ls[cols]), A, M,
+                                       len(cols), K)
+    dA = dev(A)
+    with forced_plan(qe, 8, 0):
+        for tiled in (False, True) if K % 256 == 0 else (False,):
+            assert qe.gemm_prefill_plan(M, N, K, tiled) == (8, 1)
+            prep = (lambda w, s, n: qe.w4_tiled(dev(w), dev(s), n, K)) if tiled else (lambda w, s, n: (dev(w), dev(s)))
+            plain = qe.launch_gemm_prefill_w4a16_tiled if tiled else qe.launch_gemm_prefill_w4a16
+            qkv = qe.launch_gemm_prefill_qkv_w4a16_tiled if tiled else qe.launch_gemm_prefill_qkv_w4a16
+            glu = (qe.launch_gemm_prefill_dual_gate_up_swiglu_w4a16_tiled if tiled
+                   else qe.launch_gemm_prefill_dual_gate_up_swiglu_w4a16)
+            out, outw, outg = dev(R), empty((M, wide), torch.float16), empty((M, I), torch.float16)
+            plain(*prep(qw, sc, N), dA, out, out, M, N, K)
+            assert_fp16_close(host(out), ex_p, bd_p + ulp16(acc_p) * 2.0 ** 20, ref_p, what="plain",
+                              max_floor_frac=1.0)  # the floor carries the fp16 rounding of acc
+            plain(*prep(lw, ls, wide), dA, None, outw, M, wide, K)
+            assert_fp16_close(np.ascontiguousarray(host(outw)[:, cols]), ex_w, bd_w, ref_w, what="wide")
+            glu(*prep(gq, gs, 2 * I), dA, outg, M, hidden_size=K, intermediate_size=I)
+            assert_fp16_close(host(outg), ex_g, bd_g, ref_g, what="swiglu")
+            if not tiled:  # a tiled QKV needs widths that are multiples of 32
+                outs = [empty((M, n), torch.float16) for n in dims]
+                views = [t for (w, s), n, o in zip(mats, dims, outs) for t in (*prep(w, s, n), o)]
+                qkv(qe.make_qkv_view(*views), dA, M, in_features=K, num_q_heads=3, num_kv_heads=1, head_dim=40)
+                for o, (ref, ex, bd) in zip(outs, refs_q):
+                    assert_fp16_close(host(o), ex, bd, ref, what="qkv")
