@@ -150,11 +150,56 @@ __device__ __forceinline__ qwen::qe_half8_t unpack_w4t_to_half8(uint32_t w, _Flo
                                    5, 6, 7);
 }
 
+// Four accumulator elements of a fragment: elements 4 part .. 4 part + 3, with
+// SwiGLU the two element pairs (2 part + e, 2 part + e + 8) whose gate and up
+// values two neighbouring lanes exchange.  Arithmetic of epilogue_frag.
+template <int MODE>
+__device__ __forceinline__ int part_element(int part, int e) {
+    return MODE == kSwiglu ? 2 * part + (e & 1) + 8 * (e >> 1) : 4 * part + e;
+}
+
+template <int MODE>
+__device__ __forceinline__ void epilogue_part(const GemmParams& p, const float (&x)[4], int part, int r0, int col,
+                                              int lane) {
+    const int lrow = r0 + 4 * (lane >> 5);
+    if constexpr (MODE == kSwiglu) {
+        const bool gate = (lane & 1) == 0;
+        const int row0 = lrow + (gate ? 0 : 16);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float lo = x[e], hi = x[e + 2];
+            const float lo_x = swap_adjacent(lo), hi_x = swap_adjacent(hi);
+            const int v = 2 * part + e, row = row0 + 8 * (v >> 2) + (v & 3);
+            if (col < p.N && row < p.M)
+                p.out[0][static_cast<size_t>(row) * p.out_stride[0] + (col >> 1)] =
+                    f2h(silu_mul(gate ? lo : hi_x, gate ? lo_x : hi));
+        }
+        return;
+    }
+    if (col >= p.N) return;
+    int m = 0, local = col;
+    if constexpr (MODE == kQKV) {
+        m = (col >= p.col_begin[1]) + (col >= p.col_begin[2]);
+        local = col - p.col_begin[m];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int row = lrow + 8 * part + e;
+        if (row >= p.M) continue;
+        const size_t off = static_cast<size_t>(row) * p.out_stride[m] + local;
+        _Float16 h = static_cast<_Float16>(x[e]);
+        if (MODE == kPlain && p.residual != nullptr) h = h + __builtin_bit_cast(_Float16, p.residual[off]);
+        p.out[m][off] = __builtin_bit_cast(uint16_t, h);
+    }
+}
+
 // Sums the K-slice partials in slice order and applies the epilogue.  grid
-// (N tiles, M tiles, fragments): block z takes the 32x32 fragment z of its
-// tile, 256 threads in the MFMA lane layout of the 4 waves.  S > 0: all S
-// slices are requested before the first add (one memory latency, not S);
-// S = 0: a loop over the slices.
+// (N tiles, M tiles, 4 * fragments): block z takes a quarter of the elements of
+// the 32x32 fragment z / 4 of its tile, 256 threads in the MFMA lane layout of
+// the 4 waves.  Bound by what a CU takes from L2, so the blocks are small: with
+// whole fragments the down projection at M = 128 (6 slices, 4.7 MB) had 48 of
+// them and took 7.5 us, now 3.1.  S slices are requested before the first add (one
+// memory latency, not S); S = 0: any number, eight at a time.
 template <int BM, int BN, int WGM, int MODE, int S>
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmParams p, int slices) {
     constexpr int WGN = 4 / WGM;
@@ -162,34 +207,33 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmParams p, i
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tile = blockIdx.y * gridDim.x + blockIdx.x;
     const int n_tiles = gridDim.x * gridDim.y;
-    const int f = blockIdx.z, i = f / NI, j = f % NI;
+    const int f = blockIdx.z >> 2, part = blockIdx.z & 3, i = f / NI, j = f % NI;
     const size_t slice_stride = static_cast<size_t>(n_tiles) * (BM * BN);
-    const float* part = p.ws + static_cast<size_t>(tile) * (BM * BN) + f * 16 * 256 + tid;
-    f32x16 acc = f32x16{};
-    if constexpr (S > 0) {
-        float x[S][16];
+    const float* src = p.ws + static_cast<size_t>(tile) * (BM * BN) + f * 16 * 256 + tid;
+    constexpr int B = S > 0 ? S : 8;
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int z0 = 0; z0 < (S > 0 ? 1 : slices); z0 += B) {
+        float x[B][4];
 #pragma unroll
-        for (int z = 0; z < S; ++z)
+        for (int z = 0; z < B; ++z)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) x[z][v] = part[z * slice_stride + v * 256];
+            for (int e = 0; e < 4; ++e)
+                x[z][e] = src[(S > 0 ? z : min(z0 + z, slices - 1)) * slice_stride + part_element<MODE>(part, e) * 256];
 #pragma unroll
-        for (int z = 0; z < S; ++z)
+        for (int z = 0; z < B; ++z)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[v] += x[z][v];
-    } else {
-        for (int z = 0; z < slices; ++z)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[v] += part[z * slice_stride + v * 256];
+            for (int e = 0; e < 4; ++e)
+                if (S > 0 || z0 + z < slices) acc[e] += x[z][e];
     }
     const int wm = wave / WGN, wn = wave % WGN;
-    epilogue_frag<MODE>(p, acc, blockIdx.y * BM + wm * WM + i * 32, blockIdx.x * BN + wn * WN + j * 32 + (lane & 31),
-                        lane);
+    epilogue_part<MODE>(p, acc, part, blockIdx.y * BM + wm * WM + i * 32,
+                        blockIdx.x * BN + wn * WN + j * 32 + (lane & 31), lane);
 }
 
 template <int BM, int BN, int WGM, int MODE>
 void launch_reduce(const GemmParams& p, dim3 tiles, int slices, hipStream_t s) {
     constexpr int FR = (BM / WGM / 32) * (BN / (4 / WGM) / 32);  // fragments per wave
-    const dim3 grid(tiles.x, tiles.y, FR);
+    const dim3 grid(tiles.x, tiles.y, 4 * FR);
     switch (slices) {
         case 2: gemm_splitk_reduce_kernel<BM, BN, WGM, MODE, 2><<<grid, 256, 0, s>>>(p, slices); break;
         case 3: gemm_splitk_reduce_kernel<BM, BN, WGM, MODE, 3><<<grid, 256, 0, s>>>(p, slices); break;

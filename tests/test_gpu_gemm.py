@@ -535,3 +535,35 @@ def test_gemm_few_rows(qe, orc, M, K):
                 qkv(qe.make_qkv_view(*views), dA, M, in_features=K, num_q_heads=3, num_kv_heads=1, head_dim=40)
                 for o, (ref, ex, bd) in zip(outs, refs_q):
                     assert_fp16_close(host(o), ex, bd, ref, what="qkv")
+
+
+@pytest.mark.parametrize("slices", [2, 5, 9])  # one batch of a known count, part of a batch of eight, two batches
+@pytest.mark.parametrize("tile", [1, 4])
+def test_gemm_split_k_reduce(qe, orc, tile, slices):
+    """The slice sum in quarters of a fragment: every mode, rows and columns that end inside a tile."""
+    M, N, K = 70, 200, 256 * 12
+    A = _A(orc, M, K, 91)
+    qw, sc = orc.synth_w4(92, N, K)
+    R = orc.synth_f16_normal(93, M * N).reshape(M, N)
+    dims = (128, 40, 40)
+    mats = [orc.synth_w4(94 + i, n, K) for i, n in enumerate(dims)]
+    plain, res, glu = empty((M, N), torch.float16), dev(R), empty((M, N // 2), torch.float16)
+    qkv = [empty((M, n), torch.float16) for n in dims]
+    with forced_plan(qe, tile, slices):
+        assert qe.gemm_prefill_plan(M, N, K) == (tile, slices)
+        qe.launch_gemm_prefill_w4a16(dev(qw), dev(sc), dev(A), None, plain, M, N, K)
+        qe.launch_gemm_prefill_w4a16(dev(qw), dev(sc), dev(A), res, res, M, N, K)
+        qe.launch_gemm_prefill_dual_gate_up_swiglu_w4a16(dev(qw), dev(sc), dev(A), glu, M, hidden_size=K,
+                                                         intermediate_size=N // 2)
+        w = [(dev(a), dev(b)) for a, b in mats]
+        view = qe.make_qkv_view(*w[0], qkv[0], *w[1], qkv[1], *w[2], qkv[2])
+        qe.launch_gemm_prefill_qkv_w4a16(view, dev(A), M, in_features=K, num_q_heads=16, num_kv_heads=5, head_dim=8)
+    ref, ex, bd = orc.gemm_w4a16(qw, sc, A, M, N, K)
+    assert_fp16_close(host(plain), ex, bd, ref, what=f"tile {tile} slices {slices}")
+    # the residual is added to the rounded sum, in fp16
+    assert np.array_equal(host(res).view(np.uint16), (host(plain) + R).astype(np.float16).view(np.uint16))
+    ref, ex, bd = orc.gemm_swiglu_w4a16(qw, sc, A, M, K, N // 2)
+    assert_fp16_close(host(glu), ex, bd, ref, what=f"swiglu tile {tile} slices {slices}")
+    for i, (o, n) in enumerate(zip(qkv, dims)):
+        ref, ex, bd = orc.gemm_w4a16(*mats[i], A, M, n, K)
+        assert_fp16_close(host(o), ex, bd, ref, what=f"qkv {i} tile {tile} slices {slices}")
