@@ -56,21 +56,70 @@ __global__ __launch_bounds__(256) void argmax_stage1_kernel(const uint16_t* __re
 
 // Stage 2: one block reduces nparts partials (sampling.cu:111-205) and
 // advances the control block: token_id, seq_pos + 1, rng_seed + golden ratio.
+// Latency only: the partials of a thread and the control block are requested
+// together (P per thread; a repeated last partial changes nothing), the waves
+// reduce with DPP (the largest value, then the lowest index that holds it; -0
+// and +0 compare equal, NaN is never stored).  768 partials 3.5 us as a
+// loop of dependent compares and LDS permutes, now 2.6.
+__device__ __forceinline__ int seg_min64(int v) {
+    v = min(v, qwen::dpp_i32<0xB1>(v));
+    v = min(v, qwen::dpp_i32<0x4E>(v));
+    v = min(v, qwen::dpp_i32<0x141>(v));
+    v = min(v, qwen::dpp_i32<0x140>(v));
+    v = min(v, __builtin_bit_cast(int, qwen::swz_xor16_f32(__builtin_bit_cast(float, v))));
+    return min(v, __shfl_xor(v, 32));
+}
+
+template <int P>
 __global__ __launch_bounds__(256) void argmax_stage2_advance_kernel(const float* __restrict__ val,
                                                                     const int32_t* __restrict__ idx, int nparts,
                                                                     qe_device_control_block* d_control,
                                                                     int32_t* d_pinned) {
-    Best b{-1e30f, 0};
-    for (int i = threadIdx.x; i < nparts; i += 256) b = better(b, Best{val[i], idx[i]});
-    b = block_best(b);
-    if (threadIdx.x == 0) {
-        if (d_control) {
-            d_control->token_id = b.i;
-            d_control->seq_pos += 1;
-            d_control->rng_seed += 0x9E3779B97F4A7C15ull;
-        }
-        if (d_pinned) *d_pinned = b.i;
+    int32_t seq_pos = 0;
+    uint64_t seed = 0;
+    if (d_control) {
+        seq_pos = d_control->seq_pos;
+        seed = d_control->rng_seed;
     }
+    Best b{-1e30f, 0};
+    for (int i0 = 0; i0 < nparts; i0 += 256 * P) {
+        float v[P];
+        int32_t x[P];
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            const int i = min(i0 + 256 * j + static_cast<int>(threadIdx.x), nparts - 1);
+            v[j] = val[i];
+            x[j] = idx[i];
+        }
+#pragma unroll
+        for (int j = 0; j < P; ++j) b = better(b, Best{v[j], x[j]});
+    }
+    __shared__ float s_v[4];
+    __shared__ int32_t s_i[4];
+    const float wv = qwen::seg_max<64>(b.v);
+    const int wi = seg_min64(b.v == wv ? b.i : 0x7FFFFFFF);
+    if ((threadIdx.x & 63) == 0) {
+        s_v[threadIdx.x >> 6] = wv;
+        s_i[threadIdx.x >> 6] = wi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        Best r{s_v[0], s_i[0]};
+        for (int w = 1; w < 4; ++w) r = better(r, Best{s_v[w], s_i[w]});
+        if (d_control) {
+            d_control->token_id = r.i;
+            d_control->seq_pos = seq_pos + 1;
+            d_control->rng_seed = seed + 0x9E3779B97F4A7C15ull;
+        }
+        if (d_pinned) *d_pinned = r.i;
+    }
+}
+
+void launch_stage2(const float* val, const int32_t* idx, int nparts, qe_device_control_block* ctl, int32_t* pinned,
+                   hipStream_t s) {
+    if (nparts <= 256) argmax_stage2_advance_kernel<1><<<1, 256, 0, s>>>(val, idx, nparts, ctl, pinned);
+    else if (nparts <= 768) argmax_stage2_advance_kernel<3><<<1, 256, 0, s>>>(val, idx, nparts, ctl, pinned);
+    else argmax_stage2_advance_kernel<8><<<1, 256, 0, s>>>(val, idx, nparts, ctl, pinned);
 }
 
 }  // namespace
@@ -82,7 +131,7 @@ using namespace qe;
 namespace qe {
 int launch_sample_stage2(const float* val, const int32_t* idx, int nparts, qe_device_control_block* d_control,
                          int32_t* d_pinned, hipStream_t stream) {
-    argmax_stage2_advance_kernel<<<1, 256, 0, stream>>>(val, idx, nparts, d_control, d_pinned);
+    launch_stage2(val, idx, nparts, d_control, d_pinned, stream);
     return QE_OK;
 }
 }  // namespace qe
@@ -95,7 +144,6 @@ extern "C" int qe_launch_sample_and_advance(const uint16_t* logits, float* sampl
     constexpr int kParts = 256;
     argmax_stage1_kernel<<<kParts, 256, 0, stream>>>(logits, vocab_size, sample_scratch_val, sample_scratch_idx,
                                                      d_control);
-    argmax_stage2_advance_kernel<<<1, 256, 0, stream>>>(sample_scratch_val, sample_scratch_idx, kParts, d_control,
-                                                        d_mapped_pinned_token);
+    launch_stage2(sample_scratch_val, sample_scratch_idx, kParts, d_control, d_mapped_pinned_token, stream);
     return check_launch("sample_and_advance");
 }
