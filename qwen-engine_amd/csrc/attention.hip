@@ -796,38 +796,56 @@ __global__ __launch_bounds__(256 * KG, 2) void prefill_attention_kernel(PrefillA
 }
 
 // Merges the splits of every row: 32 lanes a row (4 dims each), 8 rows a
-// block and pass.  Rows whose block of 128 had one split are already written.
+// block.  Rows whose block of 128 had one split are already written.  Lane s of
+// a row reads the (max, sum) of split s, and the partial outputs are requested
+// eight splits at a time, so a row waits for two rounds of loads: 1024 rows on
+// 15000 positions (5 splits, 31 MB) 9.4 us with a loop over the splits, now 7.0.
 __global__ __launch_bounds__(256) void prefill_attention_combine_kernel(PrefillAttnParams p) {
+    static_assert(kPaMaxSplits <= 32, "a lane per split");
     const int rows = p.T * p.group;
-    const int d = 4 * (threadIdx.x & 31);
+    const int s_lane = threadIdx.x & 31, d = 4 * s_lane;
     const int base = p.ctl != nullptr ? p.ctl->seq_pos : 0;
     const int all = rows * p.nkv;
-    for (int i = blockIdx.x * 8 + (threadIdx.x >> 5); i < all; i += gridDim.x * 8) {
-        const int kvh = i / rows, r = i - kvh * rows;
-        const int live = prefill_live_splits(prefill_tiles(r / kPaRows, rows, p.group, base, p.max_seq), p.splits);
-        if (live == 1) continue;
-        float m = -INFINITY;
-        for (int s = 0; s < live; ++s) m = fmaxf(m, p.part_ml[2 * (static_cast<size_t>(s) * all + i)]);
-        float l = 0.0f;
-        float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        for (int s = 0; s < live; ++s) {
-            const size_t row = static_cast<size_t>(s) * all + i;
-            const float2 ml = *reinterpret_cast<const float2*>(p.part_ml + 2 * row);
-            const float w = ml.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml.x - m);
-            const float4 v = *reinterpret_cast<const float4*>(p.part_o + row * kHeadDim + d);
-            l += w * ml.y;
-            o.x += w * v.x;
-            o.y += w * v.y;
-            o.z += w * v.z;
-            o.w += w * v.w;
+    const int i = blockIdx.x * 8 + (threadIdx.x >> 5);
+    if (i >= all) return;
+    const int kvh = i / rows, r = i - kvh * rows;
+    const int live = prefill_live_splits(prefill_tiles(r / kPaRows, rows, p.group, base, p.max_seq), p.splits);
+    if (live == 1) return;
+    constexpr int B = 8;
+    float2 ml = make_float2(-INFINITY, 0.0f);
+    if (s_lane < live)
+        ml = *reinterpret_cast<const float2*>(p.part_ml + 2 * (static_cast<size_t>(s_lane) * all + i));
+    float4 v[B];
+    auto request = [&](int s0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+            v[b] = *reinterpret_cast<const float4*>(
+                p.part_o + (static_cast<size_t>(min(s0 + b, live - 1)) * all + i) * kHeadDim + d);
+    };
+    request(0);
+    const float m = qwen::seg_max<32>(ml.x);
+    const float w_lane = ml.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml.x - m);
+    float l = 0.0f;
+    float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int s0 = 0; s0 < live; s0 += B) {
+        if (s0 > 0) request(s0);
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            if (s0 + b >= live) break;
+            const float w = __shfl(w_lane, s0 + b, 32);
+            l += w * __shfl(ml.y, s0 + b, 32);
+            o.x += w * v[b].x;
+            o.y += w * v[b].y;
+            o.z += w * v[b].z;
+            o.w += w * v[b].w;
         }
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-        uint16_t* dst =
-            p.out + static_cast<size_t>(r / p.group) * p.out_stride + (kvh * p.group + r % p.group) * kHeadDim + d;
-        *reinterpret_cast<uint2*>(dst) =
-            make_uint2(static_cast<uint32_t>(f2h(o.x * inv)) | (static_cast<uint32_t>(f2h(o.y * inv)) << 16),
-                       static_cast<uint32_t>(f2h(o.z * inv)) | (static_cast<uint32_t>(f2h(o.w * inv)) << 16));
     }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    uint16_t* dst =
+        p.out + static_cast<size_t>(r / p.group) * p.out_stride + (kvh * p.group + r % p.group) * kHeadDim + d;
+    *reinterpret_cast<uint2*>(dst) =
+        make_uint2(static_cast<uint32_t>(f2h(o.x * inv)) | (static_cast<uint32_t>(f2h(o.y * inv)) << 16),
+                   static_cast<uint32_t>(f2h(o.z * inv)) | (static_cast<uint32_t>(f2h(o.w * inv)) << 16));
 }
 
 }  // namespace
@@ -990,8 +1008,7 @@ int launch_prefill_attention(const uint16_t* q, const uint16_t* layer_k_cache, c
     else
         prefill_attention_kernel<1, true><<<static_cast<unsigned>(blocks * p.splits), 256, 0, stream>>>(p);
     if (p.splits > 1)
-        prefill_attention_combine_kernel<<<static_cast<unsigned>(std::min((rows * num_kv_heads + 7) / 8, 4LL * cus)), 256,
-                                           0, stream>>>(p);
+        prefill_attention_combine_kernel<<<static_cast<unsigned>((rows * num_kv_heads + 7) / 8), 256, 0, stream>>>(p);
     return check_launch("attention_gqa_prefill");
 }
 
