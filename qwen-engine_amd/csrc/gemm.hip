@@ -666,183 +666,40 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, Workspace ws
     return check_launch(what);
 }
 
-// ---- W4A8 variant: int8 activations on the int8 matrix cores ----------------------
-// v_mfma_i32_32x32x32_i8 takes 16 int8 k per lane; within one 128-group a
-// lane half h covers k in [64h, 64h + 64), 16 per MFMA j (k = 64h + 16j), for
-// both operands.  The weights enter as their unsigned nibbles q (two ops per
-// 4 bytes: & 0x0F0F0F0F and >> 4); sum (q - 8) a = sum q a + the Q8_1 sum8
-// terms (-8 * sum a per 8 elements), so the correction per row and group is
-// the sum of its 16 sum8 words.  Per group: 4 MFMAs into an int32 tile from
-// zero, then fp32 += float(int dot + correction) * (w_scale * x_scale) - the
-// GEMV's per-chunk arithmetic with the four chunk dots summed first (integer
-// addition; evaluated as w_s * (float(dot) * x_s + float(corr) * x_s), two
-// fused multiply-adds per element and group).  A (Q8_1 int8 rows) and the
-// per-row group scale/correction go through LDS; weights straight from
-// global as in the fp16 kernel; K split into slices when the tile grid leaves
-// CUs idle (partials reduced by the fp16 kernel's reduce pass).
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x16 __attribute__((ext_vector_type(16)));
-constexpr int A8_STRIDE = 144;  // bytes per LDS row of the int8 A tile (128 + 16 pad)
-
-template <int BM, int MODE>
-__global__ __launch_bounds__(256, 2) void gemm_w4a8_mfma_kernel(GemmParams p) {
-    constexpr int BN = 128, WGM = 1, MI = BM / 32;
-    constexpr int A_U = BM / 32;  // 16-byte A chunks per thread per step: 8 threads per 128-byte row, 32 rows per pass
-    constexpr int D = 2;          // stages of the register ring
-    __shared__ __align__(16) int8_t sA[2][BM * A8_STRIDE];
-    __shared__ __align__(16) float s_xs[2][BM];
-    __shared__ __align__(16) float s_cr[2][BM];  // float(correction) * x_scale
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wn = tid >> 6;
-    const int m0 = blockIdx.y * BM;
-    const int n0 = blockIdx.x * BN;
-    const int K = p.K;
-    const int G = K >> 7;
-    const int slices = gridDim.z;
-    const int g_begin = static_cast<int>((static_cast<long long>(blockIdx.z) * G) / slices);
-    const int g_end = static_cast<int>((static_cast<long long>(blockIdx.z + 1) * G) / slices);
-    const int KT = g_end - g_begin;  // one 128-group per step
-    const int fr = lane & 31;
-    const int h = lane >> 5;
-
-    const int a_row = tid >> 3, a_c = tid & 7;
-    const int8_t* a_src[A_U];
-#pragma unroll
-    for (int i = 0; i < A_U; ++i)
-        a_src[i] = p.A8 + static_cast<size_t>(min(m0 + a_row + 32 * i, p.M - 1)) * K + 16 * a_c;
-    const int srow = tid % BM;  // row whose group scale / correction this thread fetches
-    const size_t srow_g = static_cast<size_t>(min(m0 + srow, p.M - 1));
-    // B: the lane's column; columns past N read column N-1
-    const int col = min(n0 + wn * 32 + fr, p.N - 1);
-    int m = 0, local = col;
-    if constexpr (MODE == kQKV) {
-        m = (col >= p.col_begin[1]) + (col >= p.col_begin[2]);
-        local = col - p.col_begin[m];
+// ---- W4A8 variant: int8 activations on the int8 matrix cores (gemm_w4a8.hip) --------
+// Rows per block and K slices, from a sweep over M in {8..1500} at the
+// Qwen2.5-1.5B shapes.  128 rows where the grid has several rounds of blocks
+// (gate/up at M = 1500 93 us against 110 with 64 rows; at 512 43 against 41) or
+// where few tiles have a long K (down at M = 512 24.5 against 25.7, at 1024 37
+// against 42; at 300 20.5 against 20.1).  Slices: one block per CU where that fills
+// the chip (down at M = 300 4 slices 20.1 us, 8 21.0); else two per CU if a slice
+// keeps 12 groups (down at M = 1024 5 slices 37 us, 2 42; O at M = 1024 2 slices
+// 15.7, unsplit 11.9).  A slice has at least 3 groups, a sum at most 16 slices.
+void plan_w4a8(int M, int N, int K, size_t ws_floats, int& bm, int& slices) {
+    const int cus = cu_count(), G = K / 128;
+    const auto tiles_of = [&](int rows) { return static_cast<long long>((N + 127) / 128) * ((M + rows - 1) / rows); };
+    const long long t128 = tiles_of(128);
+    bm = t128 >= 4 * cus || (t128 <= cus && t128 * G >= 12 * cus) ? 128 : 64;
+    const long long tiles = tiles_of(bm);
+    slices = 1;
+    if (tiles < cus && gemm_split_k_enabled()) {
+        const int one = static_cast<int>(cus / tiles), two = static_cast<int>(2 * cus / tiles);
+        slices = 20 * one * tiles < 17 * cus && G >= 12 * two ? two : one;
+        slices = std::min({slices, G / 3, 16});
     }
-    const u32x4* b_src = reinterpret_cast<const u32x4*>(p.qw[m] + static_cast<size_t>(local) * (K >> 3)) + 2 * h;
-    const uint16_t* b_sc = p.sc[m] + static_cast<size_t>(local) * G;
-
-    struct Stage {
-        i32x4 a[A_U];
-        float xs;
-        i32x4 s8[4];
-        u32x4 b[2];
-        uint32_t bs;
-    };
-    Stage st[D];
-    auto load = [&](int kt, Stage& S) __attribute__((always_inline)) {
-        const int g = g_begin + kt;
-#pragma unroll
-        for (int i = 0; i < A_U; ++i) S.a[i] = *reinterpret_cast<const i32x4*>(a_src[i] + g * 128);
-        S.xs = p.A8_scale[srow_g * G + g];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            S.s8[j] = *reinterpret_cast<const i32x4*>(p.A8_sum8 + srow_g * (K >> 3) + 16 * g + 4 * j);
-        S.b[0] = b_src[4 * g];  // cached: every M tile of the column reads it
-        S.b[1] = b_src[4 * g + 1];
-        S.bs = b_sc[g];
-    };
-    auto store = [&](int buf, const Stage& S) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < A_U; ++i)
-            *reinterpret_cast<i32x4*>(&sA[buf][(a_row + 32 * i) * A8_STRIDE + 16 * a_c]) = S.a[i];
-        int cr = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) cr += S.s8[j].x + S.s8[j].y + S.s8[j].z + S.s8[j].w;
-        s_xs[buf][srow] = S.xs;  // threads srow and srow + BM write the same values
-        s_cr[buf][srow] = static_cast<float>(cr) * S.xs;
-    };
-
-    f32x16 f[MI][1];
-#pragma unroll
-    for (int i = 0; i < MI; ++i) f[i][0] = f32x16{};
-
-#pragma unroll
-    for (int d = 0; d < D; ++d) load(min(d, KT - 1), st[d]);
-    store(0, st[0]);
-    __syncthreads();
-
-    auto step = [&](int kt, int d) __attribute__((always_inline)) {
-        const int buf = kt & 1;
-        const Stage& S = st[d];
-        i32x16 acc[MI];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t w0 = S.b[j >> 1][(2 * j) & 3], w1 = S.b[j >> 1][(2 * j + 1) & 3];
-            const i32x4 bop = {static_cast<int>(w0 & 0x0F0F0F0Fu), static_cast<int>((w0 >> 4) & 0x0F0F0F0Fu),
-                               static_cast<int>(w1 & 0x0F0F0F0Fu), static_cast<int>((w1 >> 4) & 0x0F0F0F0Fu)};
-#pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                const i32x4 aop =
-                    *reinterpret_cast<const i32x4*>(&sA[buf][(i * 32 + fr) * A8_STRIDE + 64 * h + 16 * j]);
-                acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop, bop, j == 0 ? i32x16{} : acc[i], 0, 0, 0);
-            }
-        }
-        const float ws = h2f(static_cast<uint16_t>(S.bs));
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-#pragma unroll
-            for (int v4 = 0; v4 < 4; ++v4) {
-                const int r0 = i * 32 + 8 * v4 + 4 * h;  // rows r0..r0+3 hold elements 4*v4 .. 4*v4+3
-                const f32x4 xs4 = *reinterpret_cast<const f32x4*>(&s_xs[buf][r0]);
-                const f32x4 cr4 = *reinterpret_cast<const f32x4*>(&s_cr[buf][r0]);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {  // f += w_s * (float(dot) * x_s + float(corr) * x_s)
-                    const int v = 4 * v4 + q;
-                    f[i][0][v] = fmaf(ws, fmaf(static_cast<float>(acc[i][v]), xs4[q], cr4[q]), f[i][0][v]);
-                }
-            }
-        }
-        load(min(kt + D, KT - 1), st[d]);  // step kt is consumed: refill with step kt + D
-        store(buf ^ 1, st[(d + 1) % D]);   // step kt + 1, loaded D - 1 steps ago
-        __syncthreads();
-    };
-    int kt = 0;
-    for (; kt + D <= KT; kt += D) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) step(kt + d, d);
-    }
-    if (kt < KT) step(kt, 0);  // tail (D = 2)
-    if (slices == 1) {
-        epilogue<BM, BN, WGM, MODE>(p, f, m0, n0, 0, wn, lane);
-        return;
-    }
-    const int tile = blockIdx.y * gridDim.x + blockIdx.x;
-    const int n_tiles = gridDim.x * gridDim.y;
-    float* mine = p.ws + (static_cast<size_t>(blockIdx.z) * n_tiles + tile) * (BM * BN);
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) mine[(i * 16 + v) * 256 + tid] = f[i][0][v];
+    if (const int f = gemm_forced_slices()) slices = f;
+    slices = std::max(1, std::min(slices, G));
+    while (slices > 1 && static_cast<size_t>(slices) * tiles * bm * 128 > ws_floats) --slices;
 }
 
 template <int MODE>
 int launch_gemm_w4a8(GemmParams p, hipStream_t stream, const char* what, Workspace ws) {
     if (p.M <= 0 || p.N <= 0) return QE_OK;
     p.ws = ws.ptr;
-    const size_t ws_floats = ws.ptr == nullptr ? 0 : ws.floats;
-    // 128-row tiles when they already give one block per CU, else 64-row tiles
-    const int cus = cu_count();
-    const int nt128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
-    const bool big = nt128 >= cus;
-    const int bm = big ? 128 : 64;
+    int bm, slices;
+    plan_w4a8(p.M, p.N, p.K, ws.ptr == nullptr ? 0 : ws.floats, bm, slices);
     if ((p.M + bm - 1) / bm > 65535) return fail(QE_ERR_UNSUPPORTED, "%s: M=%d too large", what, p.M);
-    const dim3 grid((p.N + 127) / 128, (p.M + bm - 1) / bm);
-    const int tiles = static_cast<int>(grid.x * grid.y);
-    const int G = p.K / 128;
-    int slices = 1;  // about two blocks per CU, >= 4 groups per slice
-    if (tiles < cus && gemm_split_k_enabled()) slices = std::max(1, std::min((2 * cus + tiles - 1) / tiles, G / 4));
-    if (const int f = gemm_forced_slices()) slices = std::max(1, std::min(f, G));
-    while (slices > 1 && static_cast<size_t>(slices) * tiles * bm * 128 > ws_floats) --slices;
-    const dim3 g3(grid.x, grid.y, slices);
-    if (big) gemm_w4a8_mfma_kernel<128, MODE><<<g3, 256, 0, stream>>>(p);
-    else gemm_w4a8_mfma_kernel<64, MODE><<<g3, 256, 0, stream>>>(p);
-    if (slices > 1) {
-        if (big) launch_reduce<128, 128, 1, MODE>(p, grid, slices, stream);
-        else launch_reduce<64, 128, 1, MODE>(p, grid, slices, stream);
-    }
+    launch_gemm_w4a8(MODE, bm, p, slices, stream);
     return check_launch(what);
 }
 

@@ -251,6 +251,9 @@ void launch_reduce(const GemmParams& p, dim3 tiles, int slices, hipStream_t s) {
 // k groups a block; p.ws holds the partials when slices > 1.
 void launch_gemm_dma(int mode, int tile, const GemmParams& p, int slices, hipStream_t stream);
 
+// W4A8 (gemm_w4a8.hip): bm 64 or 128 rows a block; p.ws holds the partials when slices > 1.
+void launch_gemm_w4a8(int mode, int bm, const GemmParams& p, int slices, hipStream_t stream);
+
 // The kernel for up to kSkinnyRows rows (gemm_skinny.hip).
 constexpr int kSkinnyRows = 32;
 inline int skinny_columns(int M, int N) { return M <= 16 && N >= 16 * 512 ? 32 : 16; }  // of a block

@@ -567,3 +567,42 @@ def test_gemm_split_k_reduce(qe, orc, tile, slices):
     for i, (o, n) in enumerate(zip(qkv, dims)):
         ref, ex, bd = orc.gemm_w4a16(*mats[i], A, M, n, K)
         assert_fp16_close(host(o), ex, bd, ref, what=f"qkv {i} tile {tile} slices {slices}")
+
+
+@pytest.mark.parametrize("M,N,K,slices", [(129, 1541, 15232, 0),  # 128-row blocks; more groups than ring stages
+                                          (70, 131, 2304, 9),     # two batches of the slice sum
+                                          (3, 7, 256, 2),         # one group a slice
+                                          (65, 260, 384, 1)])     # stores of four, fewer groups than ring stages + 1
+def test_gemm_w4a8_edges(qe, orc, M, N, K, slices):
+    """Rows and columns that end inside a block, matrix boundaries inside a store of four, odd SwiGLU widths."""
+    A = _A(orc, M, K, 21)
+    q8, xs, s8 = _q8_rows(qe, A)
+    qw, sc = orc.synth_w4(22 + N, N, K)
+    R = orc.synth_f16_normal(23, M * N).reshape(M, N)
+    out, res = empty((M, N), torch.float16), dev(R)
+    I = (N - 1) // 2
+    glu = empty((M, I), torch.float16)
+    dims = (27, 6, 6)
+    mats = [orc.synth_w4(24 + i, n, K) for i, n in enumerate(dims)]
+    w = [(dev(a), dev(b)) for a, b in mats]
+    qkv = [empty((M, n), torch.float16) for n in dims]
+    view = qe.make_qkv_view(*w[0], qkv[0], *w[1], qkv[1], *w[2], qkv[2])
+    with forced_plan(qe, 0, slices):
+        qe.launch_gemm_prefill_w4a8(dev(qw), dev(sc), q8, xs, s8, None, out, M, N, K)
+        qe.launch_gemm_prefill_w4a8(dev(qw), dev(sc), q8, xs, s8, res, res, M, N, K)
+        qe.launch_gemm_prefill_dual_gate_up_swiglu_w4a8(dev(qw), dev(sc), q8, xs, s8, glu, M, hidden_size=K,
+                                                        intermediate_size=I)
+        qe.launch_gemm_prefill_qkv_w4a8(view, q8, xs, s8, M, in_features=K, num_q_heads=9, num_kv_heads=2, head_dim=3)
+    rows = sorted({0, 1, M // 2, M - 2, M - 1} | set(range(min(30, M), min(34, M))))
+    ref, ex, bd = _rows_ref(orc, qw, sc, q8, xs, s8, rows, N, K)
+    what = f"w4a8 {M}x{N}x{K} slices {slices}"
+    assert_fp16_close(host(out)[rows], ex, bd, ref, what=what)
+    assert np.array_equal(host(res).view(np.uint16), (host(out) + R).astype(np.float16).view(np.uint16)), what
+    g, u = ex[:, 0:2 * I:2], ex[:, 1:2 * I:2]
+    # silu(g) u moves by at most 1.1 |u| dg + |silu(g)| du; dg, du: the fp32 sums, 2^-20 of sum |terms|
+    silu = g / (1 + np.exp(-g))
+    bound = 1.1 * np.abs(u) * bd[:, 0:2 * I:2] + np.abs(silu) * bd[:, 1:2 * I:2]
+    assert_fp16_close(host(glu)[rows], silu * u, bound, what=what + " swiglu")
+    for (a, b), o, n in zip(mats, qkv, dims):
+        ref, ex, bd = _rows_ref(orc, a, b, q8, xs, s8, rows, n, K)
+        assert_fp16_close(host(o)[rows], ex, bd, ref, what=what + " qkv")
