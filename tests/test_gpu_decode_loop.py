@@ -308,7 +308,7 @@ def test_engine_prefill_lm_head_matches_oracle(qe, orc):
     (21, 0, 12, 2, 512, True), (22, 511, 12, 2, 4096, True), (64, 448, 12, 2, 2048, True), (509, 0, 12, 2, 4096, True),
     (43, 1500, 12, 2, 4096, True), (43, 1500, 12, 2, 4096, False), (300, 1800, 8, 8, 2100, True),
     (5, 2043, 7, 1, 2048, True), (30, 2030, 12, 2, 2048, True), (1100, 0, 32, 32, 1100, True),
-    (1100, 60, 32, 32, 1200, False), (2, 300, 64, 1, 512, True)])
+    (1100, 60, 32, 32, 1200, False), (2, 300, 64, 1, 512, True), (17, 4000, 12, 2, 4096, True)])
 def test_prefill_attention_splits_and_groups(qe, T, base, nq, nkv, max_seq, ws, shift):
     """Row blocks, key splits (with and without a stream workspace) and the two
     key groups (more than one block per CU) against float64; the cache past the

@@ -155,3 +155,18 @@ def test_rmsnorm_kernels_agree_bit_for_bit(qe, orc, H):
             assert np.array_equal(host(norm).view(np.uint16), a[t].view(np.uint16)), t
     ref = orc.rmsnorm_fp16(x16, g16)
     assert np.all(np.abs(a.astype(np.float64) - ref.astype(np.float64)) <= ulp_or_zero(ref))
+
+
+@pytest.mark.parametrize("H", [8, 504, 1024, 1032, 1536, 2048, 2056, 4096, 4104])  # edges of the units a lane holds
+@pytest.mark.parametrize("T", [1, 258])  # one row a block; four, the last block half full (256 CUs)
+def test_rmsnorm_fp16_widths(qe, orc, H, T):
+    rng = np.random.default_rng(H + T)
+    x16 = rng.standard_normal((T, H)).astype(np.float16)
+    g16 = (1 + 0.2 * rng.standard_normal(H)).astype(np.float16)
+    out, x = empty((T + 1, H), torch.float16).fill_(7.0), dev(x16)
+    qe.launch_rmsnorm_fp16(x, dev(g16), out, T, hidden_size=H)
+    got, ref = host(out), orc.rmsnorm_fp16(x16, g16)
+    assert np.all(np.abs(got[:T].astype(np.float64) - ref.astype(np.float64)) <= ulp_or_zero(ref))
+    assert np.all(got[T] == 7.0)  # nothing past the last row
+    qe.launch_rmsnorm_fp16(x, dev(g16), x, T, hidden_size=H)  # in place
+    assert np.array_equal(host(x).view(np.uint16), got[:T].view(np.uint16))
