@@ -166,10 +166,13 @@ int qe_gemm_release_workspace(hipStream_t stream);
  * process (only qe_gemm_reserve_workspace makes them).  Test hook. */
 long qe_gemm_workspace_allocations(void);
 
-/* The tile (1 64x64, 2 64x128, 3 128x64, 4 128x128) and K-slice count a
- * prefill GEMM of this shape would use on the current device with a stream
- * workspace (tiled != 0: the tiled-layout launchers), after the qe_set_tuning
- * overrides.  Host only; no counterpart in the reference. */
+/* The tile (1 64x64, 2 64x128, 3 128x64, 4 128x128) and K-slice count of the
+ * register-staged kernels for a prefill GEMM of this shape on the current
+ * device with a stream workspace (tiled != 0: the tiled-layout launchers),
+ * after the qe_set_tuning overrides (gemm_tile 5..8 is reported as set).  The
+ * launchers take this plan, or a kernel for few rows or for tiled weights
+ * through LDS where that is predicted to be faster.  Host only; no counterpart
+ * in the reference. */
 int qe_gemm_prefill_plan(int M, int N, int K, int tiled, int* tile, int* slices);
 
 /* Replaces launch_gemm_prefill_w4a16, include/kernels.cuh:119-130.

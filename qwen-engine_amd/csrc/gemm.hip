@@ -585,7 +585,8 @@ float predict_skinny_us(int M, int N, int K, bool tiled, int cus) {
 // 2048 19.6 against 25) and lose 1 to 6 us on shorter ones (QKV at M = 512 15.7
 // against 10.0).  The register-staged model is 10 % low around the crossing and
 // 15 to 25 % low past M = 1280, hence the factors.
-void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& slices) {
+// staged_only: among the register-staged tiles, as qe_gemm_prefill_plan reports.
+void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& slices, bool staged_only = false) {
     const int cus = cu_count();
     const int KT = K / BK;
     const int max_slices = (K % 256 == 0) ? KT / 4 : KT;  // QUAD slices whole 256-k quads
@@ -607,7 +608,7 @@ void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& 
             if (us < best) { best = us; ti = i; slices = s; }
         }
     }
-    if (tiled && M > 64) {
+    if (tiled && M > 64 && !staged_only) {
         best *= M >= 1280 ? 1.25f : 1.12f;
         for (int i = 4; i < 4 + kDmaTiles; ++i) {
             for (int s : {1, 2, 3, 4, 6}) {
@@ -620,7 +621,7 @@ void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& 
     }
     // a few rows: the tile model is 5 to 15 % high there (gate/up 10.0 against
     // 10.5 us predicted, down 12.0 against 14.0, tiled)
-    const bool few = M <= kSkinnyRows && gemm_forced_slices() == 0 &&
+    const bool few = !staged_only && M <= kSkinnyRows && gemm_forced_slices() == 0 &&
                      predict_skinny_us(M, N, K, tiled, cus) < 0.9f * best;
     if (few) {
         ti = kSkinnyTile;
@@ -973,7 +974,7 @@ extern "C" int qe_launch_gemm_prefill_w4a16_noalloc(const uint32_t* qweight, con
 extern "C" int qe_gemm_prefill_plan(int M, int N, int K, int tiled, int* tile, int* slices) {
     QE_REQUIRE(M > 0 && N > 0 && K > 0 && K % 128 == 0 && tile && slices, "gemm_prefill_plan: bad arguments");
     int ti = 0, s = 1;
-    plan_gemm(M, N, K, kWsFloats, tiled != 0, ti, s);
+    plan_gemm(M, N, K, kWsFloats, tiled != 0, ti, s, true);
     *tile = ti + 1;
     *slices = s;
     return QE_OK;

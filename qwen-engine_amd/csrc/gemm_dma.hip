@@ -10,9 +10,10 @@ namespace {
 //
 // A 64-k step is one stage of a ring of D in LDS: the A tile (BM rows of 128
 // bytes) and the packed words of the block's columns.  A row's 16-byte chunk ch
-// (k 8 ch .. 8 ch + 7 of the step) is stored at ch ^ (row / 2 % 8), so the
-// 16-byte operand reads of 16 rows touch every bank once.  Lane half h takes
-// k 32 h + 8 s in sub-step s.  Words and scales of a wave's columns are
+// is stored at ch ^ (row / 2 % 8), so the 16-byte operand reads of 16 rows touch
+// every bank once.  Step t of a 256-k quad takes k 128 h + 32 t + 8 s for lane half
+// h in sub-step s (chunk ch = 4 h + s), the order of the register-staged kernels:
+// an unsplit sum has their bits, whichever the planner picks.  Words and scales of a wave's columns are
 // requested and read by that wave alone (WGM = 1); only A is shared.
 // KG = 2: two groups of four waves, each with a ring of its own, take half of
 // the block's k each and add their accumulators through LDS at the end (one
@@ -87,11 +88,11 @@ __global__ __launch_bounds__(256 * KG, 2) void gemm_w4a16_dma_kernel(GemmParams 
     for (int i = 0; i < LA; ++i) {
         const int row = 8 * (4 * i + wave) + (lane >> 3);
         const int ch = (lane & 7) ^ ((row >> 1) & 7);
-        a_off[i] = static_cast<uint32_t>(min(m0 + row, p.M - 1) - m0) * (2 * K) + 16 * ch;
+        a_off[i] = static_cast<uint32_t>(min(m0 + row, p.M - 1) - m0) * (2 * K) + 16 * (ch & 3) + 256 * (ch >> 2);
     }
     const char* a_base = reinterpret_cast<const char*>(p.A + static_cast<size_t>(m0) * K + 256 * q_safe);
     // words: 1 KB of a 32-column tile per step; columns past N read the last tile
-    const uint32_t b_off = 1024 * h + 16 * fr;
+    const uint32_t b_off = 16 * lane;
     const char* b_base[NI];
     const char* s_ptr = nullptr;  // this lane's 4 bytes of scales: lanes 0..31 tile 0, 32..63 tile 1
 #pragma unroll
@@ -111,12 +112,12 @@ __global__ __launch_bounds__(256 * KG, 2) void gemm_w4a16_dma_kernel(GemmParams 
 
     auto load_stage = [&](int kt, int slot) __attribute__((always_inline)) {
         const uint32_t st = lds0 + slot * STAGE;
-        const char* ab = a_base + static_cast<size_t>(kt) * 128;
+        const char* ab = a_base + static_cast<size_t>(kt >> 2) * 512 + 64 * (kt & 3);
 #pragma unroll
         for (int i = 0; i < LA; ++i)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                          ::"s"(st + (4 * i + wave) * 1024), "v"(a_off[i]), "s"(ab) : "memory");
-        const size_t bk = static_cast<size_t>(kt >> 2) * 4096 + 2048 * (kt & 1) + 512 * ((kt >> 1) & 1);
+        const size_t bk = static_cast<size_t>(kt >> 2) * 4096 + 1024 * (kt & 3);
 #pragma unroll
         for (int j = 0; j < NI; ++j)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
@@ -151,7 +152,7 @@ __global__ __launch_bounds__(256 * KG, 2) void gemm_w4a16_dma_kernel(GemmParams 
         for (int j = 0; j < NI; ++j) {
             w[j] = *reinterpret_cast<l_u32x4>(st + A_BYTES + (wn * NI + j) * 1024 + 16 * lane);
             sc[j] = __builtin_bit_cast(_Float16, *reinterpret_cast<l_u16>(sc_lds + ((kt >> 2) & 3) * 256 + j * 128 +
-                                                                         ((kt >> 1) & 1) * 64 + 2 * fr));
+                                                                         64 * h + 2 * fr));
         }
     };
     auto read_a = [&](uint32_t st, int s, int i) __attribute__((always_inline)) {
