@@ -986,7 +986,8 @@ int launch_prefill_attention(const uint16_t* q, const uint16_t* layer_k_cache, c
     // the stream's workspace for their partials, and the context has tiles;
     // a row block then takes as many of them as its own tiles are worth.
     const int cus = cu_count();
-    const StreamWorkspace ws = stream_workspace(stream);
+    const WorkspaceLease lease(stream);  // until both kernels are enqueued
+    const StreamWorkspace ws = lease.ws;
     const long long part = rows * num_kv_heads * (kHeadDim + 2);  // floats of one split
     p.splits = 1;
     // (contexts below 16 tiles: the second launch costs what the splits save)

@@ -634,6 +634,7 @@ void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& 
     while (slices > 1 && !fits(ti, slices)) --slices;
 }
 
+// ws: the caller's for the whole call (WorkspaceLease, a temporary of the calling expression)
 template <int MODE>
 int launch_gemm(GemmParams p, hipStream_t stream, const char* what, Workspace ws, bool tiled = false) {
     if (p.M <= 0 || p.N <= 0) return QE_OK;
@@ -749,8 +750,15 @@ __global__ __launch_bounds__(256) void repack_w4_tiled_kernel(const u32x4* __res
 // never holds a workspace (its GEMMs run unsplit); the null stream is the one
 // legacy stream of the device (this library is built without per-thread
 // default streams), shared correctly ordered by every thread.
+//
+// Two locks.  A slot's `launch` mutex is held while a launch that uses the
+// slot's workspace is enqueued (WorkspaceLease) and while the slot changes;
+// g_ws_mutex guards the table itself and is only ever taken last.  Slots keep
+// their place, so a slot's mutex can be waited for without the table's; who
+// gets it looks again whether the slot still is that stream's.
 constexpr int kMaxWsStreams = 64;
 struct WsSlot {
+    bool used;
     hipStream_t stream;
     float* ptr;
     size_t floats;
@@ -758,38 +766,49 @@ struct WsSlot {
 };
 std::mutex g_ws_mutex;
 WsSlot g_ws[64][kMaxWsStreams];
-int g_ws_count[64];
+std::mutex g_ws_launch[64][kMaxWsStreams];
+int g_ws_top[64];  // slots from here on were never used
 std::atomic<long> g_ws_allocations{0};  // hipMalloc calls made for workspaces
 
 bool per_thread_handle(hipStream_t stream) { return stream == hipStreamPerThread; }
 
-Workspace gemm_workspace(hipStream_t stream) {
-    if (!gemm_split_k_enabled() || per_thread_handle(stream)) return {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
-        (void)hipGetLastError();
-        return {};
-    }
-    std::lock_guard<std::mutex> lock(g_ws_mutex);
-    for (int i = 0; i < g_ws_count[dev]; ++i)
-        if (g_ws[dev][i].stream == stream) return {g_ws[dev][i].ptr, g_ws[dev][i].floats};
-    return {};
+// The slot of `stream`, -1 without one; the caller holds g_ws_mutex.
+int ws_find(int dev, hipStream_t stream) {
+    for (int i = 0; i < g_ws_top[dev]; ++i)
+        if (g_ws[dev][i].used && g_ws[dev][i].stream == stream) return i;
+    return -1;
 }
 
-// registers (ptr, floats) for `stream` on the current device; the caller
-// holds g_ws_mutex.  Returns the slot or nullptr when the table is full.
-WsSlot* ws_find_or_add(int dev, hipStream_t stream, bool* found) {
-    for (int i = 0; i < g_ws_count[dev]; ++i)
-        if (g_ws[dev][i].stream == stream) {
-            *found = true;
-            return &g_ws[dev][i];
+// Both locks of a stream's slot; the table's alone when it has none (slot -1).
+struct WsLocked {
+    std::unique_lock<std::mutex> launch, table;
+    int slot = -1;
+    WsLocked(int dev, hipStream_t stream) {
+        for (;;) {
+            table = std::unique_lock<std::mutex>(g_ws_mutex);
+            const int want = ws_find(dev, stream);
+            if (want == slot) return;
+            table.unlock();
+            if (launch.owns_lock()) launch.unlock();
+            if (want >= 0) launch = std::unique_lock<std::mutex>(g_ws_launch[dev][want]);
+            slot = want;
         }
-    *found = false;
-    if (g_ws_count[dev] == kMaxWsStreams) return nullptr;
-    WsSlot* s = &g_ws[dev][g_ws_count[dev]++];
-    *s = WsSlot{stream, nullptr, 0, false};
-    return s;
-}
+    }
+    // The slot to register a workspace in: the stream's own or a free one, -1 when all are taken.
+    int place(int dev) const {
+        if (slot >= 0) return slot;
+        int i = 0;
+        while (i < g_ws_top[dev] && g_ws[dev][i].used) ++i;
+        return i < kMaxWsStreams ? i : -1;
+    }
+    // Registers it; returns the workspace the library owned there, to be freed.
+    float* put(int dev, int i, const WsSlot& workspace) {
+        float* old = slot >= 0 && g_ws[dev][i].owned ? g_ws[dev][i].ptr : nullptr;
+        g_ws_top[dev] = std::max(g_ws_top[dev], i + 1);
+        g_ws[dev][i] = workspace;
+        return old;
+    }
+};
 
 int current_device(const char* what, int* dev) {
     if (hipGetDevice(dev) != hipSuccess || *dev < 0 || *dev >= 64) {
@@ -801,7 +820,18 @@ int current_device(const char* what, int* dev) {
 
 }  // namespace
 
-StreamWorkspace stream_workspace(hipStream_t stream) { return gemm_workspace(stream); }
+WorkspaceLease::WorkspaceLease(hipStream_t stream) {
+    if (!gemm_split_k_enabled() || per_thread_handle(stream)) return;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
+        (void)hipGetLastError();
+        return;
+    }
+    WsLocked s(dev, stream);
+    if (s.slot < 0) return;
+    ws = {g_ws[dev][s.slot].ptr, g_ws[dev][s.slot].floats};
+    launch_ = std::move(s.launch);
+}
 
 }  // namespace qe
 
@@ -817,13 +847,12 @@ extern "C" int qe_gemm_reserve_workspace(hipStream_t stream) {
         return qe::fail(QE_ERR_HIP, "%s: invalid stream", what);
     }
     QE_REQUIRE(st == hipStreamCaptureStatusNone, "%s: stream is capturing", what);
-    std::lock_guard<std::mutex> lock(qe::g_ws_mutex);
-    bool found = false;
-    qe::WsSlot* s = qe::ws_find_or_add(dev, stream, &found);
-    if (s == nullptr)
+    qe::WsLocked s(dev, stream);
+    const int i = s.place(dev);
+    if (i < 0)
         return qe::fail(QE_ERR_UNSUPPORTED, "%s: %d streams already hold a workspace on this device", what,
                         qe::kMaxWsStreams);
-    if (found && s->floats >= qe::kWsFloats) {
+    if (s.slot >= 0 && qe::g_ws[dev][i].floats >= qe::kWsFloats) {
         qe::clear_error();
         return QE_OK;
     }
@@ -831,11 +860,10 @@ extern "C" int qe_gemm_reserve_workspace(hipStream_t stream) {
     ++qe::g_ws_allocations;
     if (hipMalloc(&ptr, qe::kWsFloats * sizeof(float)) != hipSuccess) {
         (void)hipGetLastError();
-        if (!found) --qe::g_ws_count[dev];
         return qe::fail(QE_ERR_HIP, "%s: hipMalloc of %zu bytes failed", what, qe::kWsFloats * sizeof(float));
     }
-    if (found && s->owned) (void)hipFree(s->ptr);
-    *s = qe::WsSlot{stream, static_cast<float*>(ptr), qe::kWsFloats, true};
+    if (float* old = s.put(dev, i, qe::WsSlot{true, stream, static_cast<float*>(ptr), qe::kWsFloats, true}))
+        (void)hipFree(old);
     qe::clear_error();
     return QE_OK;
 }
@@ -848,14 +876,14 @@ extern "C" int qe_gemm_attach_workspace(hipStream_t stream, void* workspace, siz
     QE_REQUIRE(bytes >= (size_t(1) << 20), "%s: %zu bytes is below the 1 MiB minimum", what, bytes);
     int dev = 0;
     QE_TRY(qe::current_device(what, &dev));
-    std::lock_guard<std::mutex> lock(qe::g_ws_mutex);
-    bool found = false;
-    qe::WsSlot* s = qe::ws_find_or_add(dev, stream, &found);
-    if (s == nullptr)
+    qe::WsLocked s(dev, stream);
+    const int i = s.place(dev);
+    if (i < 0)
         return qe::fail(QE_ERR_UNSUPPORTED, "%s: %d streams already hold a workspace on this device", what,
                         qe::kMaxWsStreams);
-    if (found && s->owned) (void)hipFree(s->ptr);
-    *s = qe::WsSlot{stream, static_cast<float*>(workspace), std::min(bytes / sizeof(float), qe::kWsFloats), false};
+    if (float* old = s.put(dev, i, qe::WsSlot{true, stream, static_cast<float*>(workspace),
+                                              std::min(bytes / sizeof(float), qe::kWsFloats), false}))
+        (void)hipFree(old);
     qe::clear_error();
     return QE_OK;
 }
@@ -863,13 +891,10 @@ extern "C" int qe_gemm_attach_workspace(hipStream_t stream, void* workspace, siz
 extern "C" int qe_gemm_release_workspace(hipStream_t stream) {
     int dev = 0;
     QE_TRY(qe::current_device("gemm_release_workspace", &dev));
-    std::lock_guard<std::mutex> lock(qe::g_ws_mutex);
-    for (int i = 0; i < qe::g_ws_count[dev]; ++i)
-        if (qe::g_ws[dev][i].stream == stream) {
-            if (qe::g_ws[dev][i].owned) (void)hipFree(qe::g_ws[dev][i].ptr);
-            qe::g_ws[dev][i] = qe::g_ws[dev][--qe::g_ws_count[dev]];
-            break;
-        }
+    qe::WsLocked s(dev, stream);
+    if (s.slot >= 0) {
+        if (float* old = s.put(dev, s.slot, qe::WsSlot{})) (void)hipFree(old);
+    }
     qe::clear_error();
     return QE_OK;
 }
@@ -886,6 +911,7 @@ namespace {
 // only that address (the array's name is not a device address on the host).
 __device__ __align__(256) float scratch[kWsFloats];
 std::mutex g_scratch_mutex;
+std::mutex g_scratch_launch[64];  // held while a launch that uses a device's scratch is enqueued
 float* g_scratch_ptr[64];
 
 float* scratch_address(int dev) {
@@ -933,7 +959,7 @@ extern "C" int qe_launch_gemm_prefill_w4a16(const uint32_t* qweight, const uint1
     p.M = M;
     p.N = N;
     p.K = K;
-    return launch_gemm<kPlain>(p, stream, what, gemm_workspace(stream));
+    return launch_gemm<kPlain>(p, stream, what, WorkspaceLease(stream).ws);
 }
 
 extern "C" int qe_launch_gemm_prefill_w4a16_noalloc(const uint32_t* qweight, const uint16_t* scales,
@@ -955,6 +981,7 @@ extern "C" int qe_launch_gemm_prefill_w4a16_noalloc(const uint32_t* qweight, con
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
         return fail(QE_ERR_HIP, "%s: no current device", what);
+    std::lock_guard<std::mutex> launch(g_scratch_launch[dev]);
     float* ws = gemm_split_k_enabled() ? scratch_address(dev) : nullptr;
     if (gemm_split_k_enabled() && ws == nullptr)
         return fail(QE_ERR_HIP, "%s: hipGetSymbolAddress(scratch) failed", what);
@@ -1022,7 +1049,7 @@ extern "C" int qe_launch_gemm_prefill_w4a16_tiled(const uint32_t* tiled_weight, 
     p.M = M;
     p.N = N;
     p.K = K;
-    return launch_gemm<kPlain>(p, stream, what, gemm_workspace(stream), true);
+    return launch_gemm<kPlain>(p, stream, what, WorkspaceLease(stream).ws, true);
 }
 
 extern "C" int qe_launch_gemm_prefill_qkv_w4a16_tiled(const qe_qkv_view* view, const uint16_t* input_x, int M,
@@ -1058,7 +1085,7 @@ extern "C" int qe_launch_gemm_prefill_qkv_w4a16_tiled(const qe_qkv_view* view, c
     p.M = M;
     p.N = q_dim + 2 * kv_dim;
     p.K = in_features;
-    return launch_gemm<kQKV>(p, stream, what, gemm_workspace(stream), true);
+    return launch_gemm<kQKV>(p, stream, what, WorkspaceLease(stream).ws, true);
 }
 
 extern "C" int qe_launch_gemm_prefill_dual_gate_up_swiglu_w4a16_tiled(const uint32_t* tiled_weight,
@@ -1081,7 +1108,7 @@ extern "C" int qe_launch_gemm_prefill_dual_gate_up_swiglu_w4a16_tiled(const uint
     p.M = M;
     p.N = 2 * intermediate_size;
     p.K = hidden_size;
-    return launch_gemm<kSwiglu>(p, stream, what, gemm_workspace(stream), true);
+    return launch_gemm<kSwiglu>(p, stream, what, WorkspaceLease(stream).ws, true);
 }
 
 extern "C" int qe_launch_gemm_prefill_qkv_w4a16(const qe_qkv_view* view, const uint16_t* input_x, int M,
@@ -1115,7 +1142,7 @@ extern "C" int qe_launch_gemm_prefill_qkv_w4a16(const qe_qkv_view* view, const u
     p.M = M;
     p.N = q_dim + 2 * kv_dim;
     p.K = in_features;
-    return launch_gemm<kQKV>(p, stream, what, gemm_workspace(stream));
+    return launch_gemm<kQKV>(p, stream, what, WorkspaceLease(stream).ws);
 }
 
 extern "C" int qe_launch_gemm_prefill_dual_gate_up_swiglu_w4a16(const uint32_t* gate_up_qweight,
@@ -1138,7 +1165,7 @@ extern "C" int qe_launch_gemm_prefill_dual_gate_up_swiglu_w4a16(const uint32_t* 
     p.M = M;
     p.N = 2 * intermediate_size;
     p.K = hidden_size;
-    return launch_gemm<kSwiglu>(p, stream, what, gemm_workspace(stream));
+    return launch_gemm<kSwiglu>(p, stream, what, WorkspaceLease(stream).ws);
 }
 
 // ---- W4A8 prefill GEMM entry points --------------------------------------------------
@@ -1172,7 +1199,7 @@ extern "C" int qe_launch_gemm_prefill_w4a8(const uint32_t* qweight, const uint16
     p.M = M;
     p.N = N;
     p.K = K;
-    return launch_gemm_w4a8<kPlain>(p, stream, what, gemm_workspace(stream));
+    return launch_gemm_w4a8<kPlain>(p, stream, what, WorkspaceLease(stream).ws);
 }
 
 extern "C" int qe_launch_gemm_prefill_qkv_w4a8(const qe_qkv_view* view, const int8_t* input_q8,
@@ -1208,7 +1235,7 @@ extern "C" int qe_launch_gemm_prefill_qkv_w4a8(const qe_qkv_view* view, const in
     p.M = M;
     p.N = q_dim + 2 * kv_dim;
     p.K = in_features;
-    return launch_gemm_w4a8<kQKV>(p, stream, what, gemm_workspace(stream));
+    return launch_gemm_w4a8<kQKV>(p, stream, what, WorkspaceLease(stream).ws);
 }
 
 extern "C" int qe_launch_gemm_prefill_dual_gate_up_swiglu_w4a8(const uint32_t* gate_up_qweight,
@@ -1233,5 +1260,5 @@ extern "C" int qe_launch_gemm_prefill_dual_gate_up_swiglu_w4a8(const uint32_t* g
     p.M = M;
     p.N = 2 * intermediate_size;
     p.K = hidden_size;
-    return launch_gemm_w4a8<kSwiglu>(p, stream, what, gemm_workspace(stream));
+    return launch_gemm_w4a8<kSwiglu>(p, stream, what, WorkspaceLease(stream).ws);
 }

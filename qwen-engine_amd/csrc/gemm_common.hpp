@@ -40,9 +40,9 @@ __device__ __forceinline__ float silu_mul(float g, float u) {
 
 // Split-K partials: fp32 tiles of the K slices, reduced by a second kernel
 // on the same stream (deterministic order, no atomics or fences).  They live
-// in a workspace of kWsFloats floats that belongs to the launching stream
-// (gemm_workspace below), so GEMMs in flight on different streams never
-// share partials.
+// in a workspace of at most kWsFloats floats that belongs to the launching
+// stream (WorkspaceLease), so GEMMs in flight on different streams never share
+// partials.
 constexpr size_t kWsFloats = size_t(8) << 20;  // 32 MiB
 
 using Workspace = StreamWorkspace;

@@ -7,6 +7,8 @@
 #include <stdio.h>
 #include <stdarg.h>
 
+#include <mutex>
+
 #include "qe_kernels.h"
 #include "quant_primitives.hpp"
 
@@ -32,13 +34,25 @@ int gemv_forced_cap();     // 0 auto, else the largest GEMV grid (larger grids l
 int engine_tiled_prefill();  // engines created from now on keep tiled copies for the prefill GEMMs (default 1)
 
 // The split workspace registered for a stream (qe_gemm_reserve_workspace /
-// qe_gemm_attach_workspace), {nullptr, 0} without one.  A launch may use it
-// from its first kernel to its last: later work on the stream waits for it.
+// qe_gemm_attach_workspace), {nullptr, 0} without one.
 struct StreamWorkspace {
     float* ptr = nullptr;
     size_t floats = 0;
 };
-StreamWorkspace stream_workspace(hipStream_t stream);
+
+// A stream's workspace, for the time in which one launch is enqueued.  What a
+// launch writes into it is read by a later kernel of the same launch, so both
+// are enqueued while this is held: threads that share a stream (the null stream
+// above all) take turns, and the workspace is neither replaced nor freed in
+// between.  Launches on other streams do not wait.
+class WorkspaceLease {
+public:
+    explicit WorkspaceLease(hipStream_t stream);
+    StreamWorkspace ws;
+
+private:
+    std::unique_lock<std::mutex> launch_;
+};
 
 // qe_launch_attention_gqa_prefill for callers that know a bound on the context
 // length the rows see (attention.hip).

@@ -1,0 +1,73 @@
+"""Which kernels a call launches, in which order and on whose behalf, checked
+without a GPU: the library's host code runs on a stand-in for the HIP runtime
+that records launches (launch_recorder.py)."""
+import pytest
+
+import launch_recorder
+
+
+@pytest.fixture(scope="module")
+def recorder(tmp_path_factory):
+    return launch_recorder.build(tmp_path_factory.mktemp("recorder"))
+
+
+@pytest.mark.parametrize("stream", [0, 0x5000])
+@pytest.mark.parametrize("one,other", [("attention(s)", "gemm(128, 1536, 8960, s)"),
+                                       ("gemm(128, 1536, 8960, s, True)", "attention(s)"),
+                                       ("gemm_w4a8(300, 1536, 8960, s)", "gemm_w4a8(200, 1536, 8960, s)"),
+                                       ("gemm_noalloc(128, 1536, 8960, s)", "gemm_noalloc(64, 1536, 8960, s)")])
+def test_partials_and_their_sum_stay_together(recorder, one, other, stream):
+    """Threads that share a stream (the null stream is every thread's default)
+    share its workspace: a launch's partials and the kernel that sums them are
+    enqueued with nothing of another thread's in between."""
+    launch_recorder.run(recorder, f"""
+        s = {stream}
+        reserve(s)
+        R.recorder_reset(2000)
+        go = threading.Barrier(3)
+        def work(k):
+            go.wait()
+            for i in range(4):
+                if k == 2: {one}
+                else: {other}
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+        [t.start() for t in threads]
+        [t.join() for t in threads]
+        e = events()
+        assert len(e) == 24, e  # every call here is split: two launches
+        for a, b in zip(e[::2], e[1::2]):
+            assert a.thread == b.thread, (a, b)
+            assert ("reduce" in b.kernel or "combine" in b.kernel) and a.stream == b.stream == s, (a, b)
+    """)
+
+
+def test_streams_do_not_wait_for_each_other_and_release_waits_for_a_launch(recorder):
+    """While one stream's launch is being enqueued, launches on another go on; a
+    workspace is given up only after the launch that uses it is enqueued whole."""
+    launch_recorder.run(recorder, """
+        a, b = 0x5000, 0x6000
+        reserve(a), reserve(b)
+        R.recorder_reset(0)
+        R.recorder_close(a)
+        t = threading.Thread(target=gemm, args=(128, 1536, 8960, a))
+        t.start()
+        while R.recorder_waiting() == 0:
+            time.sleep(0.001)
+        gemm(128, 1536, 8960, b)  # not held up by a's launch
+        r = threading.Thread(target=release, args=(a,))
+        r.start()
+        time.sleep(0.05)
+        assert r.is_alive() and not any(e.what == "free" for e in events())
+        R.recorder_open()
+        t.join(), r.join()
+        e = events()
+        assert [x.what for x in e] == ["launch"] * 4 + ["free"], e
+        assert [x.stream for x in e[:4]] == [a, b, b, a], e
+        gemm(128, 1536, 8960, a)  # unsplit now
+        assert len(events()) == 6
+        for i in range(63):  # freed entries serve other streams: at most 64 hold one
+            reserve(0x10000 + 16 * i)
+        assert L.qe_gemm_reserve_workspace(V(0x90000)) == 2
+        release(b)
+        reserve(0x90000)
+    """)
