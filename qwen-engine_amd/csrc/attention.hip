@@ -951,6 +951,14 @@ extern "C" int qe_launch_attention_gqa_flash_decode_combine(const float* splitk_
 
 namespace qe {
 
+// Whether launches on the stream are being recorded into a graph (or the runtime will not say).
+static bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 // Prefill attention; max_context bounds the positions the rows see (the
 // engine knows it on the host, the public entry point only max_seq_len).
 int launch_prefill_attention(const uint16_t* q, const uint16_t* layer_k_cache, const uint16_t* layer_v_cache,
@@ -995,6 +1003,8 @@ int launch_prefill_attention(const uint16_t* q, const uint16_t* layer_k_cache, c
         p.splits = static_cast<int>(std::max(1LL, std::min({static_cast<long long>(kPaMaxSplits), 2 * cus / blocks,
                                                             static_cast<long long>(ws.floats) / part,
                                                             static_cast<long long>(max_context) / (kPaKeys * kPaMinTiles)})));
+    // A graph may be replayed on any stream and after the workspace is gone: a recorded launch touches none.
+    if (p.splits > 1 && capturing(stream)) p.splits = 1;
     p.part_o = ws.ptr;
     p.part_ml = ws.ptr + p.splits * rows * num_kv_heads * kHeadDim;
     // Two key groups per block (one block per CU) once there is more than one

@@ -345,6 +345,46 @@ def test_prefill_attention_splits_and_groups(qe, T, base, nq, nkv, max_seq, ws, 
         assert (got[:, h] - ref).abs().max().item() <= 4.5 * 2.0 ** -10 + 2.0 ** -11
 
 
+def test_captured_prefill_attention_keeps_to_its_own_buffers(qe):
+    """A graph of a prefill attention captured on a stream with a workspace is
+    replayed on another stream after the workspace was given up: the former
+    workspace memory stays as it is, and every replay gives the bits of a launch
+    on a stream without one."""
+    T, base, nq, nkv, max_seq, D = 64, 1500, 12, 2, 4096, 128
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g).half()
+    q, kc, vc, ctl = rnd(T, nq * D), rnd(nkv, max_seq, D), rnd(nkv, max_seq, D), _ctl(base)
+
+    def launch(out, stream=None):
+        qe.launch_attention_gqa_prefill(q, kc, vc, out, ctl, T, stream=stream, num_q_heads=nq, num_kv_heads=nkv,
+                                        head_dim=D, max_seq_len=max_seq, hidden_size=nq * D)
+
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    ref, split, out = (empty((T, nq * D), torch.float16) for _ in range(3))
+    ws = torch.full((32 << 20,), 0xA5, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    launch(ref, s2)
+    qe.gemm_attach_workspace(ws, ws.numel(), s1)
+    launch(split, s1)
+    torch.cuda.synchronize()
+    assert not bool((ws == 0xA5).all())  # an eager launch of this shape splits its keys
+    ws.fill_(0xA5)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s1):
+        launch(out)
+    qe.gemm_release_workspace(s1)
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s2):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+    assert bool((ws == 0xA5).all())
+
+
 def test_engine_tiled_prefill_matches_qwenbin_layout(qe):
     """The engine's prefill on the tiled weight copies gives the same hidden
     rows, logits and tokens as on the .qwenbin layout for the same GEMM plan,

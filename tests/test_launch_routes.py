@@ -71,3 +71,20 @@ def test_streams_do_not_wait_for_each_other_and_release_waits_for_a_launch(recor
         release(b)
         reserve(0x90000)
     """)
+
+
+def test_recorded_prefill_attention_takes_no_workspace(recorder):
+    """A graph may be replayed on any stream and after the capturing stream's
+    workspace is released, so a launch recorded into one is a single kernel."""
+    launch_recorder.run(recorder, """
+        s = 0x5000
+        reserve(s)
+        attention(s)
+        R.recorder_set_capturing(s, 1)
+        attention(s)
+        R.recorder_set_capturing(s, 0)
+        attention(s)
+        split, combine, one, split2, combine2 = events()
+        assert "combine" in combine.kernel and (split, combine) == (split2, combine2)
+        assert one.kernel == split.kernel and one.grid[0] * 10 == split.grid[0], (one, split)
+    """)
