@@ -577,7 +577,7 @@ float predict_skinny_us(int M, int N, int K, bool tiled, int cus) {
 }
 
 // Tile and K-slice plan of a prefill GEMM: the configuration the time model
-// predicts fastest among those whose split-K partials fit ws_floats, then the
+// predicts fastest among those whose split-K partials fit ws_floats, under the
 // gemm_tile / gemm_slices overrides.  ti: 0..3 the register-staged tiles, 4..6
 // the kernels of gemm_dma.hip (tiled weights only).  Those win where a launch
 // has enough steps to fill (gate/up at M = 1024 72 against 78 us, 2048 120
@@ -585,6 +585,9 @@ float predict_skinny_us(int M, int N, int K, bool tiled, int cus) {
 // 2048 19.6 against 25) and lose 1 to 6 us on shorter ones (QKV at M = 512 15.7
 // against 10.0).  The register-staged model is 10 % low around the crossing and
 // 15 to 25 % low past M = 1280, hence the factors.
+// A forced tile takes the slice count of the best plan of its own family
+// (register-staged, LDS ring); only a launch with no tile forced is free to
+// leave the family.
 // staged_only: among the register-staged tiles, as qe_gemm_prefill_plan reports.
 void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& slices, bool staged_only = false) {
     const int cus = cu_count();
@@ -597,40 +600,39 @@ void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& 
     auto fits = [&](int i, int s) {
         return i < 4 ? fits_tile(kTiles[i].bm, kTiles[i].bn, s) : fits_tile(kDma[i - 4].bm, kDma[i - 4].bn, s);
     };
-    ti = 0;
-    slices = 1;
     float best = 1e30f;
-    for (int i = 0; i < 4; ++i) {
-        for (int s : {1, 2, 3, 4, 6}) {
-            if (s > 1 && !gemm_split_k_enabled()) break;
-            if (!fits(i, s)) continue;
-            const float us = predict_us(tiled ? kTilesTiled[i] : kTiles[i], M, N, K, s, cus);
-            if (us < best) { best = us; ti = i; slices = s; }
-        }
-    }
-    if (tiled && M > 64 && !staged_only) {
-        best *= M >= 1280 ? 1.25f : 1.12f;
-        for (int i = 4; i < 4 + kDmaTiles; ++i) {
+    auto search = [&](int first, int last) {
+        for (int i = first; i < last; ++i) {
             for (int s : {1, 2, 3, 4, 6}) {
                 if (s > 1 && !gemm_split_k_enabled()) break;
                 if (!fits(i, s)) continue;
-                const float us = predict_dma_us(kDma[i - 4], M, N, K, s, cus);
+                const float us = i < 4 ? predict_us(tiled ? kTilesTiled[i] : kTiles[i], M, N, K, s, cus)
+                                       : predict_dma_us(kDma[i - 4], M, N, K, s, cus);
                 if (us < best) { best = us; ti = i; slices = s; }
             }
         }
+    };
+    const int f = gemm_forced_tile() - 1, n = gemm_forced_slices();
+    const bool force_staged = f >= 0 && f < 4, force_dma = f >= 4 && f < 4 + kDmaTiles && tiled;
+    const bool force_few = f == kSkinnyTile && M <= kSkinnyRows;
+    const bool any = !force_staged && !force_dma && !force_few && !staged_only;
+    ti = 0;
+    slices = 1;
+    if (!force_dma) search(0, 4);
+    if (any && tiled && M > 64) {
+        best *= M >= 1280 ? 1.25f : 1.12f;
+        search(4, 4 + kDmaTiles);
     }
+    if (force_dma) search(4, 4 + kDmaTiles);
     // a few rows: the tile model is 5 to 15 % high there (gate/up 10.0 against
     // 10.5 us predicted, down 12.0 against 14.0, tiled)
-    const bool few = !staged_only && M <= kSkinnyRows && gemm_forced_slices() == 0 &&
-                     predict_skinny_us(M, N, K, tiled, cus) < 0.9f * best;
-    if (few) {
+    if (force_few || (any && M <= kSkinnyRows && n == 0 && predict_skinny_us(M, N, K, tiled, cus) < 0.9f * best)) {
         ti = kSkinnyTile;
         slices = 1;
+        return;
     }
-    const int f = gemm_forced_tile();
-    if ((f >= 1 && f <= 4) || (f >= 5 && f <= 7 && tiled) || (f == kSkinnyTile + 1 && M <= kSkinnyRows)) ti = f - 1;
-    if (const int n = gemm_forced_slices()) slices = n;
-    if (ti == kSkinnyTile) slices = 1;
+    if (force_staged || force_dma) ti = f;
+    if (n != 0) slices = n;
     while (slices > 1 && !fits(ti, slices)) --slices;
 }
 

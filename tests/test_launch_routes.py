@@ -88,3 +88,28 @@ def test_recorded_prefill_attention_takes_no_workspace(recorder):
         assert "combine" in combine.kernel and (split, combine) == (split2, combine2)
         assert one.kernel == split.kernel and one.grid[0] * 10 == split.grid[0], (one, split)
     """)
+
+
+@pytest.mark.parametrize("tiled", [False, True])
+def test_forced_tile_takes_the_slices_of_its_own_family(recorder, tiled):
+    """With gemm_tile 1..4 and no slice count forced, a launch runs what
+    qe_gemm_prefill_plan reports, also where another kernel (few rows, LDS ring)
+    would have been chosen and would have run unsplit."""
+    launch_recorder.run(recorder, f"""
+        tiled = {tiled}
+        reserve()
+        seen = set()
+        for tile, (bm, bn) in enumerate([(64, 64), (64, 128), (128, 64), (128, 128)], 1):
+            tune("gemm_tile", tile)
+            for M in (1, 9, 32, 33, 128, 200, 700, 1024, 1500, 2048):
+                for N, K in ((2048, 1536), (1536, 1536), (17920, 1536), (1536, 8960)):
+                    t, s = I(), I()
+                    ok(L.qe_gemm_prefill_plan(I(M), I(N), I(K), I(tiled), ctypes.byref(t), ctypes.byref(s)))
+                    R.recorder_reset(0)
+                    gemm(M, N, K, 0, tiled)
+                    e = events()[0]
+                    assert t.value == tile and e.grid == ((N + bn - 1) // bn, (M + bm - 1) // bm, s.value), (M, N, K, e)
+                    assert "ILi%dELi%dE" % (bm, bn) in e.kernel, e
+                    seen.add((tile, M, N, K, s.value))
+        assert (1, 9, 1536, 8960, 6) in seen and (4, 2048, 1536, 8960, 1) in seen, sorted(seen)
+    """)
