@@ -166,13 +166,19 @@ int qe_gemm_release_workspace(hipStream_t stream);
  * process (only qe_gemm_reserve_workspace makes them).  Test hook. */
 long qe_gemm_workspace_allocations(void);
 
-/* The tile (1 64x64, 2 64x128, 3 128x64, 4 128x128) and K-slice count of the
- * register-staged kernels for a prefill GEMM of this shape on the current
- * device with a stream workspace (tiled != 0: the tiled-layout launchers),
- * after the qe_set_tuning overrides (gemm_tile 5..8 is reported as set).  The
- * launchers take this plan, or a kernel for few rows or for tiled weights
- * through LDS where that is predicted to be faster.  Host only; no counterpart
- * in the reference. */
+/* The tile (1..8, the numbers of the gemm_tile switch) and K-slice count that a
+ * prefill W4A16 GEMM of this shape runs with on the current device, on a
+ * stream with a 32 MiB workspace (tiled != 0: the tiled-layout launchers),
+ * after the qe_set_tuning overrides.  A row's result depends on its inputs,
+ * the tile, the slice count and gemm_ks2 alone: rows computed in several launches
+ * equal one launch of all of them bit for bit when gemm_tile and gemm_slices
+ * are set to its plan and gemm_ks2 to 1 or 2 (tiles 1..4 only look at it).  Host
+ * only; no counterpart in the reference. */
+int qe_gemm_prefill_launch_plan(int M, int N, int K, int tiled, int* tile, int* slices);
+
+/* The same among the register-staged tiles 1..4 alone (a gemm_tile of 5..8 is
+ * reported as set): what a launch runs with under the gemm_staged switch.
+ * Without it the launchers also choose kernels 5..8, which add in another order. */
 int qe_gemm_prefill_plan(int M, int N, int K, int tiled, int* tile, int* slices);
 
 /* Replaces launch_gemm_prefill_w4a16, include/kernels.cuh:119-130.
@@ -220,10 +226,11 @@ int qe_launch_gemm_prefill_dual_gate_up_swiglu_w4a16(const uint32_t* gate_up_qwe
  * 16-byte chunks (chunk 8g + 4h + i of column c), and 64 fp16 scales as
  * [h][c] (group 2g + h of column c).  Columns are padded to a multiple of 32
  * (zeros), and each word holds its nibbles in the order the dequantization
- * reads fastest.  Requires K % 256 == 0.  For a given tile and K-slice plan
- * the results equal the .qwenbin-layout launchers' bit for bit; the plan
- * comes from a time model fitted to these kernels.  10-20 % faster on
- * MI355X at the Qwen2.5-1.5B shapes. */
+ * reads fastest.  Requires K % 256 == 0.  For a given tile of 1..4 and K-slice
+ * count the results equal the .qwenbin-layout launchers' bit for bit; the
+ * automatic plan comes from a time model fitted to these kernels and may name
+ * tiles 5..7, which exist for this layout only.  10-20 % faster on MI355X at
+ * the Qwen2.5-1.5B shapes. */
 
 /* Bytes of the tiled copy of an N x K matrix (weights, scales). */
 int qe_w4_tiled_bytes(int N, int K, size_t* weight_bytes, size_t* scale_bytes);
@@ -417,6 +424,9 @@ int qe_stream_read(const void* data, size_t bytes, uint32_t* sink, hipStream_t s
  *   32 rows (ignored for more; never sliced);
  *   "gemm_slices" 0..64 (default 0 = chosen per shape) - force the number of
  *   K slices;
+ *   "gemm_staged" 0/1 (default 0) - automatic W4A16 plans keep to tiles 1..4
+ *   (qe_gemm_prefill_plan): both weight layouts then give the same bits where
+ *   their plans agree;
  *   "gemm_ks2" 0..2 (default 0) - prefill GEMMs with K % 256 == 0 split the k
  *   steps of a block over two groups of four waves: 0 when the grid has at
  *   most one block per CU, 1 never, 2 always;

@@ -588,7 +588,7 @@ float predict_skinny_us(int M, int N, int K, bool tiled, int cus) {
 // A forced tile takes the slice count of the best plan of its own family
 // (register-staged, LDS ring); only a launch with no tile forced is free to
 // leave the family.
-// staged_only: among the register-staged tiles, as qe_gemm_prefill_plan reports.
+// staged_only (or the gemm_staged switch): among the register-staged tiles.
 void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& slices, bool staged_only = false) {
     const int cus = cu_count();
     const int KT = K / BK;
@@ -615,7 +615,7 @@ void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& 
     const int f = gemm_forced_tile() - 1, n = gemm_forced_slices();
     const bool force_staged = f >= 0 && f < 4, force_dma = f >= 4 && f < 4 + kDmaTiles && tiled;
     const bool force_few = f == kSkinnyTile && M <= kSkinnyRows;
-    const bool any = !force_staged && !force_dma && !force_few && !staged_only;
+    const bool any = !force_staged && !force_dma && !force_few && !staged_only && !gemm_staged_only();
     ti = 0;
     slices = 1;
     if (!force_dma) search(0, 4);
@@ -1004,6 +1004,15 @@ extern "C" int qe_gemm_prefill_plan(int M, int N, int K, int tiled, int* tile, i
     QE_REQUIRE(M > 0 && N > 0 && K > 0 && K % 128 == 0 && tile && slices, "gemm_prefill_plan: bad arguments");
     int ti = 0, s = 1;
     plan_gemm(M, N, K, kWsFloats, tiled != 0, ti, s, true);
+    *tile = ti + 1;
+    *slices = s;
+    return QE_OK;
+}
+
+extern "C" int qe_gemm_prefill_launch_plan(int M, int N, int K, int tiled, int* tile, int* slices) {
+    QE_REQUIRE(M > 0 && N > 0 && K > 0 && K % 128 == 0 && tile && slices, "gemm_prefill_launch_plan: bad arguments");
+    int ti = 0, s = 1;
+    plan_gemm(M, N, K, kWsFloats, tiled != 0, ti, s);
     *tile = ti + 1;
     *slices = s;
     return QE_OK;

@@ -13,11 +13,13 @@ namespace {
 // is stored at ch ^ (row / 2 % 8), so the 16-byte operand reads of 16 rows touch
 // every bank once.  Step t of a 256-k quad takes k 128 h + 32 t + 8 s for lane half
 // h in sub-step s (chunk ch = 4 h + s), the order of the register-staged kernels:
-// an unsplit sum has their bits, whichever the planner picks.  Words and scales of a wave's columns are
-// requested and read by that wave alone (WGM = 1); only A is shared.
+// with KG = 1 a slice has the bits of their kernel with one k group.  Words and
+// scales of a wave's columns are requested and read by that wave alone (WGM = 1);
+// only A is shared.
 // KG = 2: two groups of four waves, each with a ring of its own, take half of
-// the block's k each and add their accumulators through LDS at the end (one
-// block per CU; half the split-K partials for the same parallelism).
+// the block's k each and add their accumulators through LDS at the end, which is
+// another order of the sum (one block per CU; half the split-K partials for the
+// same parallelism).
 //
 // What bounds it.  The 128 x 32 wave tile of the register-staged kernels reads 1
 // KB of A per 32-cycle MFMA and wave, 128 bytes a clock per CU at the full

@@ -16,6 +16,7 @@ thread_local char g_last_error[1024] = "";
 int g_cu_count[64] = {0};
 int g_gemm_split_k = 1;
 int g_gemm_tile = 0;
+int g_gemm_staged = 0;
 int g_gemm_slices = 0;
 int g_gemm_ks2 = 0;
 int g_gemv_bt = 0;
@@ -26,6 +27,7 @@ int g_engine_tiled = 1;
 int gemm_split_k_enabled() { return g_gemm_split_k; }
 int gemm_forced_tile() { return g_gemm_tile; }
 int gemm_forced_slices() { return g_gemm_slices; }
+int gemm_staged_only() { return g_gemm_staged; }
 int gemm_ks2_mode() { return g_gemm_ks2; }
 int gemv_forced_bt() { return g_gemv_bt; }
 int gemv_forced_cap() { return g_gemv_cap; }
@@ -66,6 +68,10 @@ extern "C" int qe_set_tuning(const char* key, int value) {
     if (std::strcmp(key, "gemm_tile") == 0) {
         if (value < 0 || value > 8) return qe::fail(QE_ERR_INVALID_ARGUMENT, "set_tuning: gemm_tile %d not in 0..8", value);
         qe::g_gemm_tile = value;
+        return QE_OK;
+    }
+    if (std::strcmp(key, "gemm_staged") == 0) {
+        qe::g_gemm_staged = value != 0;
         return QE_OK;
     }
     if (std::strcmp(key, "gemv_block") == 0) {

@@ -67,6 +67,7 @@ OTHER_SIGNATURES = {
     "qe_w4_tiled_bytes": [_I, _I, ctypes.POINTER(ctypes.c_size_t), ctypes.POINTER(ctypes.c_size_t)],
     "qe_repack_w4_tiled": [_P, _P, _I, _I, _P, _P, _P],
     "qe_gemm_prefill_plan": [_I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)],
+    "qe_gemm_prefill_launch_plan": [_I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)],
 }
 
 ENGINE_SIGNATURES = {
@@ -546,9 +547,19 @@ def gemm_workspace_allocations() -> int:
 
 
 def gemm_prefill_plan(M, N, K, tiled=False):
-    """(tile, slices) a prefill GEMM of this shape would use (qe_gemm_prefill_plan)."""
+    """(tile, slices) of the register-staged kernels for a prefill GEMM of this shape: what it runs with
+    under the gemm_staged switch (qe_gemm_prefill_plan)."""
     t, sl = ctypes.c_int(), ctypes.c_int()
     _check(lib().qe_gemm_prefill_plan(M, N, K, int(tiled), ctypes.byref(t), ctypes.byref(sl)), "qe_gemm_prefill_plan")
+    return t.value, sl.value
+
+
+def gemm_prefill_launch_plan(M, N, K, tiled=False):
+    """(tile, slices) a prefill GEMM of this shape runs with on a stream with a workspace
+    (qe_gemm_prefill_launch_plan)."""
+    t, sl = ctypes.c_int(), ctypes.c_int()
+    _check(lib().qe_gemm_prefill_launch_plan(M, N, K, int(tiled), ctypes.byref(t), ctypes.byref(sl)),
+           "qe_gemm_prefill_launch_plan")
     return t.value, sl.value
 
 

@@ -99,7 +99,7 @@ def test_gemm_full_size_properties(qe, orc, tiled):
     y3 = run(np.ascontiguousarray(qw[perm]), np.ascontiguousarray(sc[perm]), A, M)
     assert np.array_equal(_bits(y3), _bits(y1)[:, perm])
     # rows in two launches with the plan of the whole launch (tile and slices forced)
-    tile, slices = qe.gemm_prefill_plan(M, N, K, tiled)
+    tile, slices = qe.gemm_prefill_launch_plan(M, N, K, tiled)
     try:
         qe.set_tuning("gemm_tile", tile)
         qe.set_tuning("gemm_slices", slices)
@@ -109,3 +109,73 @@ def test_gemm_full_size_properties(qe, orc, tiled):
         qe.set_tuning("gemm_tile", 0)
         qe.set_tuning("gemm_slices", 0)
     assert np.array_equal(np.concatenate([_bits(top), _bits(bottom)]), _bits(y1))
+
+
+@pytest.mark.parametrize("M,N,K,tiled,tile", [(1000, 1536, 1536, True, None), (1024, 17920, 1536, True, 5),
+                                              (4096, 1536, 8960, True, 6), (2048, 2048, 1536, True, 7),
+                                              (9, 1536, 8960, True, 8), (9, 17920, 1536, False, 8),
+                                              (509, 1536, 1536, False, None)])
+def test_gemm_rows_do_not_depend_on_the_launch(qe, orc, M, N, K, tiled, tile):
+    """An automatic launch equals launches of its rows in two uneven parts under
+    its own plan, for every kernel the planner chooses."""
+    got = qe.gemm_prefill_launch_plan(M, N, K, tiled)
+    print(f"gemm rows M={M} N={N} K={K} tiled={tiled} plan={got}", flush=True)
+    if tile is not None:
+        assert got[0] == tile
+    qw, sc = orc.synth_w4(61 + M, N, K)
+    w = qe.w4_tiled(dev(qw), dev(sc), N, K) if tiled else (dev(qw), dev(sc))
+    A = torch.from_numpy(orc.synth_f16_normal(62, M * K).reshape(M, K)).cuda()
+
+    def run(A_):
+        out = empty((len(A_), N), torch.float16)
+        launch = qe.launch_gemm_prefill_w4a16_tiled if tiled else qe.launch_gemm_prefill_w4a16
+        launch(*w, A_.contiguous(), None, out, len(A_), N, K)
+        return _bits(out)
+
+    cut = (2 * M) // 5
+    try:
+        qe.set_tuning("gemm_ks2", 1)
+        whole = run(A)
+        for key, value in zip(("gemm_tile", "gemm_slices"), got):
+            qe.set_tuning(key, value)
+        parts = np.concatenate([run(A[:cut]), run(A[cut:])])
+    finally:
+        for key in ("gemm_tile", "gemm_slices", "gemm_ks2"):
+            qe.set_tuning(key, 0)
+    assert np.array_equal(parts, whole)
+
+
+def test_gemm_staged_switch_gives_the_reported_plan(qe, orc):
+    """Under gemm_staged an automatic launch equals a launch forced to the plan of
+    gemm_prefill_plan, and both layouts agree where their plans do, at shapes that
+    otherwise take the few-rows and the LDS-ring kernels."""
+    for M, N, K in ((9, 1536, 8960), (2048, 2048, 1536)):
+        qw, sc = orc.synth_w4(71 + M, N, K)
+        packed = (dev(qw), dev(sc))
+        tiled = qe.w4_tiled(*packed, N, K)
+        A = torch.from_numpy(orc.synth_f16_normal(72, M * K).reshape(M, K)).cuda()
+        out = {}
+        try:
+            for forced in (False, True):
+                for name, w in (("packed", packed), ("tiled", tiled)):
+                    plan = qe.gemm_prefill_plan(M, N, K, name == "tiled")
+                    if forced:
+                        qe.set_tuning("gemm_staged", 0)
+                        qe.set_tuning("gemm_tile", plan[0])
+                        qe.set_tuning("gemm_slices", plan[1])
+                    else:
+                        qe.set_tuning("gemm_staged", 1)
+                        assert qe.gemm_prefill_launch_plan(M, N, K, name == "tiled") == plan
+                    y = empty((M, N), torch.float16)
+                    (qe.launch_gemm_prefill_w4a16_tiled if name == "tiled" else qe.launch_gemm_prefill_w4a16)(
+                        *w, A, None, y, M, N, K)
+                    out[forced, name] = _bits(y)
+                    for key in ("gemm_staged", "gemm_tile", "gemm_slices"):
+                        qe.set_tuning(key, 0)
+        finally:
+            for key in ("gemm_staged", "gemm_tile", "gemm_slices"):
+                qe.set_tuning(key, 0)
+        for name in ("packed", "tiled"):
+            assert np.array_equal(out[False, name], out[True, name]), (M, name)
+        if qe.gemm_prefill_plan(M, N, K, True) == qe.gemm_prefill_plan(M, N, K, False):
+            assert np.array_equal(out[False, "packed"], out[False, "tiled"]), M

@@ -113,3 +113,47 @@ def test_forced_tile_takes_the_slices_of_its_own_family(recorder, tiled):
                     seen.add((tile, M, N, K, s.value))
         assert (1, 9, 1536, 8960, 6) in seen and (4, 2048, 1536, 8960, 1) in seen, sorted(seen)
     """)
+
+
+# (rows, columns) of a block, by gemm_tile number
+TILES = {1: (64, 64), 2: (64, 128), 3: (128, 64), 4: (128, 128), 5: (128, 256), 6: (128, 256), 7: (128, 128)}
+
+
+@pytest.mark.parametrize("setting", ["", "gemm_staged 1", "gemm_tile 6", "gemm_tile 8", "gemm_slices 3"])
+@pytest.mark.parametrize("tiled", [False, True])
+def test_launch_plan_names_the_kernel_that_runs(recorder, tiled, setting):
+    """qe_gemm_prefill_launch_plan against the launches made: kernel, tile and
+    slices, over shapes at which the planner takes every kernel it has."""
+    launch_recorder.run(recorder, f"""
+        tiled, setting, TILES = {tiled}, {setting!r}.split(), {TILES}
+        reserve()
+        if setting:
+            tune(setting[0], int(setting[1]))
+        picked = set()
+        for M in (1, 9, 32, 33, 64, 65, 128, 300, 512, 1000, 1024, 1500, 2048, 4096):
+            for N, K in ((2048, 1536), (1536, 1536), (17920, 1536), (1536, 8960), (43, 768)):
+                t, s = I(), I()
+                ok(L.qe_gemm_prefill_launch_plan(I(M), I(N), I(K), I(tiled), ctypes.byref(t), ctypes.byref(s)))
+                tile, slices = t.value, s.value
+                R.recorder_reset(0)
+                gemm(M, N, K, 0, tiled)
+                e = events()
+                picked.add(tile)
+                assert len(e) == (1 if slices == 1 else 2), (M, N, K, e)
+                name, grid = e[0].kernel, e[0].grid
+                if tile == 8:
+                    assert "skinny" in name and slices == 1, e
+                    continue
+                bm, bn = TILES[tile]
+                rows, cols = (M + bm - 1) // bm, (N + bn - 1) // bn
+                assert "ILi%dELi%dE" % (bm, bn) in name, (tile, e)
+                if tile >= 5:
+                    assert "_dma_" in name and grid == (rows * cols, slices, 1), (tile, e)
+                    assert e[0].block == (256 if tile == 5 else 512), (tile, e)
+                else:
+                    assert ("_mfma_" in name or "_ks2_" in name) and grid == (cols, rows, slices), (tile, e)
+        if not setting:
+            assert picked >= (set((1, 2, 5, 6, 7, 8)) if tiled else set((1, 2, 8))), picked
+        if setting == ["gemm_staged", "1"]:
+            assert max(picked) <= 4, picked
+    """)
