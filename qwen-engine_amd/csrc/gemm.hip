@@ -589,7 +589,11 @@ float predict_skinny_us(int M, int N, int K, bool tiled, int cus) {
 // (register-staged, LDS ring); only a launch with no tile forced is free to
 // leave the family.
 // staged_only (or the gemm_staged switch): among the register-staged tiles.
-void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& slices, bool staged_only = false) {
+// ring: whether the LDS-ring kernels can take the operands (their scales go to
+// LDS in 4-byte pieces; a copy at an odd half stays with the kernels that read
+// single halves).
+void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& slices, bool staged_only = false,
+               bool ring = true) {
     const int cus = cu_count();
     const int KT = K / BK;
     const int max_slices = (K % 256 == 0) ? KT / 4 : KT;  // QUAD slices whole 256-k quads
@@ -613,13 +617,13 @@ void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& 
         }
     };
     const int f = gemm_forced_tile() - 1, n = gemm_forced_slices();
-    const bool force_staged = f >= 0 && f < 4, force_dma = f >= 4 && f < 4 + kDmaTiles && tiled;
+    const bool force_staged = f >= 0 && f < 4, force_dma = f >= 4 && f < 4 + kDmaTiles && tiled && ring;
     const bool force_few = f == kSkinnyTile && M <= kSkinnyRows;
     const bool any = !force_staged && !force_dma && !force_few && !staged_only && !gemm_staged_only();
     ti = 0;
     slices = 1;
     if (!force_dma) search(0, 4);
-    if (any && tiled && M > 64) {
+    if (any && tiled && ring && M > 64) {
         best *= M >= 1280 ? 1.25f : 1.12f;
         search(4, 4 + kDmaTiles);
     }
@@ -643,7 +647,8 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, Workspace ws
     p.ws = ws.ptr;
     const size_t ws_floats = ws.ptr == nullptr ? 0 : ws.floats;
     int ti = 0, slices = 1;
-    plan_gemm(p.M, p.N, p.K, ws_floats, tiled, ti, slices);
+    const bool ring = aligned(p.sc[0], 4) && aligned(p.sc[1], 4) && aligned(p.sc[2], 4);
+    plan_gemm(p.M, p.N, p.K, ws_floats, tiled, ti, slices, false, ring);
     if (ti == kSkinnyTile) {
         launch_gemm_skinny(MODE, p, tiled, stream);
         return check_launch(what);

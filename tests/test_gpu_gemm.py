@@ -490,6 +490,28 @@ def test_gemm_tiled_dma_tiles_ragged(qe, orc, tile, K):
         assert_fp16_close(host(outg), ex_g, bd_g, ref_g, what="swiglu " + what)
 
 
+def test_gemm_tiled_scales_at_an_odd_half(qe, orc):
+    """Tiled scales one half off the start of their buffer: the bits of the staged
+    kernels on aligned scales, at a shape the LDS-ring kernels take otherwise."""
+    M, N, K = 1024, 8192, 1536
+    assert qe.gemm_prefill_launch_plan(M, N, K, True)[0] >= 5
+    qw, sc = orc.synth_w4(740, N, K)
+    A = _A(orc, M, K, 18)
+    tw, ts = qe.w4_tiled(dev(qw), dev(sc), N, K)
+    off = torch.empty(ts.numel() + 1, dtype=ts.dtype, device="cuda")
+    off[1:] = ts.flatten()
+    got, ref = empty((M, N), torch.float16), empty((M, N), torch.float16)
+    qe.launch_gemm_prefill_w4a16_tiled(tw, off[1:], dev(A), None, got, M, N, K)
+    qe.set_tuning("gemm_staged", 1)
+    try:
+        qe.launch_gemm_prefill_w4a16_tiled(tw, ts, dev(A), None, ref, M, N, K)
+    finally:
+        qe.set_tuning("gemm_staged", 0)
+    assert np.array_equal(host(got).view(np.uint16), host(ref).view(np.uint16))
+    want, ex, bd = orc.gemm_w4a16(qw, sc, A[:4], 4, N, K)
+    assert_fp16_close(host(got)[:4], ex, bd, want, what="scales at an odd half")
+
+
 @pytest.mark.parametrize("K", [128, 384, 768, 4096])  # one group, odd groups, whole lines, several rounds a wave
 @pytest.mark.parametrize("M", [1, 16, 17, 32])
 def test_gemm_few_rows(qe, orc, M, K):

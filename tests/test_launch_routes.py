@@ -157,3 +157,31 @@ def test_launch_plan_names_the_kernel_that_runs(recorder, tiled, setting):
         if setting == ["gemm_staged", "1"]:
             assert max(picked) <= 4, picked
     """)
+
+
+@pytest.mark.parametrize("tile", [0, 5, 6, 7])
+def test_tiled_scales_at_an_odd_half_take_the_staged_kernels(recorder, tile):
+    """Tiled scales need 2-byte alignment only. The LDS-ring kernels fetch them in
+    4-byte pieces and are not chosen, nor forced, for others."""
+    launch_recorder.run(recorder, f"""
+        tune("gemm_tile", {tile})
+        for M in (1024, 2048, 4096):
+            R.recorder_reset(0)
+            gemm(M, 17920, 1536, 0, True)
+            gemm(M, 17920, 1536, 0, True, P + 2)
+            gemm(M, 17920, 1536, 0, True, P + 4)
+            a, b, c = events()
+            assert "_dma_" in a.kernel and a[2:] == c[2:], (a, c)
+            assert "_mfma_" in b.kernel or "_ks2_" in b.kernel, b
+        class View(ctypes.Structure):
+            _fields_ = [(n, V) for n in ("qw", "qs", "q", "kw", "ks", "k", "vw", "vs", "v")]
+        for odd in ("qs", "ks", "vs"):
+            R.recorder_reset(0)
+            for shift in (0, 2):
+                v = View(*[P] * 9)
+                setattr(v, odd, P + shift)
+                ok(L.qe_launch_gemm_prefill_qkv_w4a16_tiled(ctypes.byref(v), V(P), I(2048), V(0), I(1536), I(12), I(2),
+                                                            I(128)))
+            ring, staged = events()
+            assert "_dma_" in ring.kernel and "_dma_" not in staged.kernel, (ring, staged)
+    """)
