@@ -512,6 +512,9 @@ __global__ __launch_bounds__(256 * KG, 2) void prefill_attention_kernel(PrefillA
     const int lim = min(min(base + qi, p.max_seq - 1), run_end);  // last key this row takes here
     // keys every row of the wave takes: tiles that end at or before it skip the mask
     const int wave_lim = min(min(base + min(rb * kPaRows + wave * 32, rows - 1) / p.group, p.max_seq - 1), run_end);
+    // the last key that any row of the wave takes here
+    const int wave_last =
+        min(min(base + min(rb * kPaRows + wave * 32 + 31, rows - 1) / p.group, p.max_seq - 1), run_end);
     const int key_max = max(0, min(base + p.T, p.max_seq) - 1);  // the last key that holds anything
     constexpr float kScale = 1.4426950408889634f * 0.08838834764831845f;  // log2(e) / sqrt(128)
 
@@ -722,7 +725,10 @@ __global__ __launch_bounds__(256 * KG, 2) void prefill_attention_kernel(PrefillA
         mask(t, s0);
         renew_ref(row_max(s0));
         tile_barrier();  // K buffer 0 is read
-        int left = n;
+        // Tiles past the wave's last key are not multiplied: they would add nothing but 0 * V, which is NaN where
+        // a later position holds an infinity or NaN.
+        const int mine = wave_last < t * kPaKeys ? 0 : min(n, (wave_last / kPaKeys - t) / KG + 1);
+        int left = mine;
         for (; left > 2; left -= 2) {
             step(t, 0, s0, s1);
             step(t + KG, 1, s1, s0);
@@ -731,8 +737,13 @@ __global__ __launch_bounds__(256 * KG, 2) void prefill_attention_kernel(PrefillA
         if (left == 2) {
             step(t, 0, s0, s1);
             finish(1, s1);
-        } else {
+        } else if (left == 1) {
             finish(0, s0);
+        }
+        for (int i = max(mine - 1, 0); i < n - 1; ++i) {  // the tiles of the other waves
+            load_tile(vhead, it0 + kg + (i + 1) * KG, 2 + ((i & 1) ^ 1));
+            load_tile(khead, it0 + kg + (i + 2) * KG, i & 1);
+            tile_barrier();
         }
     }
     lsum += __shfl_xor(lsum, 32);

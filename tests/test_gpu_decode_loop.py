@@ -345,6 +345,46 @@ def test_prefill_attention_splits_and_groups(qe, T, base, nq, nkv, max_seq, ws, 
         assert (got[:, h] - ref).abs().max().item() <= 4.5 * 2.0 ** -10 + 2.0 ** -11
 
 
+@pytest.mark.parametrize("T,base,nq,nkv,max_seq,ws", [
+    (300, 0, 8, 8, 512, False), (200, 70, 12, 2, 512, False), (64, 1500, 8, 8, 4096, True),
+    (1500, 0, 24, 24, 1536, False), (600, 33, 64, 64, 640, False)])  # the last two: two key groups a block
+def test_prefill_attention_infinity_at_a_later_position(qe, T, base, nq, nkv, max_seq, ws):
+    """An infinity in V reaches the rows that see its position and at most the
+    rows of the same 32 queries, or of queries whose last key lies in the same 64
+    keys; every other row keeps its bits."""
+    D = 128
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T + base)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g).half()
+    q, kc, vc = rnd(T, nq * D), rnd(nkv, max_seq, D), rnd(nkv, max_seq, D)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+
+    def run(v):
+        out = empty((T, nq * D), torch.float16)
+        torch.cuda.synchronize()
+        qe.launch_attention_gqa_prefill(q, kc, v, out, _ctl(base), T, stream=s, num_q_heads=nq, num_kv_heads=nkv,
+                                        head_dim=D, max_seq_len=max_seq, hidden_size=nq * D)
+        s.synchronize()
+        return out
+
+    if ws:
+        qe.gemm_reserve_workspace(s)
+    clean = run(vc)
+    rows = torch.arange(T, device="cuda")
+    last = base + ((rows // 32 + 1) * 32).clamp(max=T)  # keys the 32 queries of a row see
+    reach = (last + 63) // 64 * 64
+    for j in range(40, T, 97):
+        v = vc.clone()
+        v[:, base + j] = float("inf")
+        got = run(v)
+        far = reach <= base + j
+        assert torch.equal(got[far].view(torch.int16), clean[far].view(torch.int16)), j
+        assert torch.isinf(got[j:]).all(), j
+    if ws:
+        qe.gemm_release_workspace(s)
+
+
 def test_captured_prefill_attention_keeps_to_its_own_buffers(qe):
     """A graph of a prefill attention captured on a stream with a workspace is
     replayed on another stream after the workspace was given up: the former
