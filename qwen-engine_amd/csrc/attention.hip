@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "attn_common.hpp"
+#include "lds_dma.hpp"
 #include "rope_common.hpp"
 
 namespace qe {
@@ -534,9 +535,7 @@ __global__ __launch_bounds__(256 * KG, 2) void prefill_attention_kernel(PrefillA
     const uint16_t* vhead = p.vc + hb;
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
                               (__attribute__((address_space(3))) void*)smem)) + kg * 4 * kPaTileBytes;
-    // Tile t into buffer `buf` (0, 1: K; 2, 3: V).  Written out: the compiler
-    // cannot tell which buffer a load in flight fills and would wait for it at
-    // the next read of LDS; tile_barrier holds the waits.
+    // Tile t into buffer `buf` (0, 1: K; 2, 3: V); tile_barrier holds the waits.
     auto load_tile = [&](const uint16_t* head, int t, int buf) __attribute__((always_inline)) {
         const uint32_t dst = lds0 + buf * kPaTileBytes + wave * 1024;
         if constexpr (!DMA) {
@@ -548,17 +547,12 @@ __global__ __launch_bounds__(256 * KG, 2) void prefill_attention_kernel(PrefillA
         } else if ((t + 1) * kPaKeys - 1 <= key_max) {  // uniform: one scalar address, one lane offset
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                             ::"s"(dst + 4096 * i), "v"(loff),
-                             "s"(head + (static_cast<size_t>(t) * kPaKeys + 16 * i) * kHeadDim)
-                             : "memory");
+                lds_load_x4(dst + 4096 * i, head + (static_cast<size_t>(t) * kPaKeys + 16 * i) * kHeadDim, loff);
         } else {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int key = min(t * kPaKeys + 16 * i + lrow, key_max);
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                             ::"s"(dst + 4096 * i), "v"(head + static_cast<size_t>(key) * kHeadDim + lcol)
-                             : "memory");
+                lds_load_x4(dst + 4096 * i, head + static_cast<size_t>(key) * kHeadDim + lcol);
             }
         }
     };

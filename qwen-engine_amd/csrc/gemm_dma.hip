@@ -1,6 +1,7 @@
 // Prefill W4A16 dequant-GEMM on tiled weights, both operands through LDS by DMA
 // (gfx950).  Math and epilogues as in gemm.hip.
 #include "gemm_common.hpp"
+#include "lds_dma.hpp"
 
 namespace qe {
 namespace {
@@ -117,17 +118,14 @@ __global__ __launch_bounds__(256 * KG, 2) void gemm_w4a16_dma_kernel(GemmParams 
         const char* ab = a_base + static_cast<size_t>(kt >> 2) * 512 + 64 * (kt & 3);
 #pragma unroll
         for (int i = 0; i < LA; ++i)
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                         ::"s"(st + (4 * i + wave) * 1024), "v"(a_off[i]), "s"(ab) : "memory");
+            lds_load_x4(st + (4 * i + wave) * 1024, ab, a_off[i]);
         const size_t bk = static_cast<size_t>(kt >> 2) * 4096 + 1024 * (kt & 3);
 #pragma unroll
         for (int j = 0; j < NI; ++j)
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                         ::"s"(st + A_BYTES + (wn * NI + j) * 1024), "v"(b_off), "s"(b_base[j] + bk) : "memory");
+            lds_load_x4(st + A_BYTES + (wn * NI + j) * 1024, b_base[j] + bk, b_off);
     };
     auto load_scales = [&](int q) __attribute__((always_inline)) {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
-                     ::"s"(sc_lds + (q & 3) * 256), "v"(s_ptr + static_cast<size_t>(q) * 128) : "memory");
+        lds_load_dword(sc_lds + (q & 3) * 256, s_ptr + static_cast<size_t>(q) * 128);
     };
     typedef const __attribute__((address_space(3))) f16x8* l_f16x8;
     typedef const __attribute__((address_space(3))) u32x4* l_u32x4;

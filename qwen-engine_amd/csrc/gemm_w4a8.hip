@@ -31,6 +31,7 @@
 #include <algorithm>
 
 #include "gemm_common.hpp"
+#include "lds_dma.hpp"
 
 namespace qe {
 namespace {
@@ -144,16 +145,12 @@ __global__ __launch_bounds__(256, 2) void gemm_w4a8_kernel(GemmParams p) {
         const uint32_t st = lds0 + slot * STAGE;
 #pragma unroll
         for (int i = 0; i < LA; ++i)
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                         ::"s"(st + (4 * i + wave) * 1024), "v"(a_src[i] + 128 * kt) : "memory");
+            lds_load_x4(st + (4 * i + wave) * 1024, a_src[i] + 128 * kt);
 #pragma unroll
         for (int b = 0; b < 2; ++b)
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                         ::"s"(st + A_BYTES + wave * 2048 + b * 1024), "v"(b_src[b] + 64 * kt) : "memory");
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
-                     ::"s"(st + A_BYTES + B_BYTES + wave * 256), "v"(xs_src + 4 * kt) : "memory");
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, off"
-                     ::"s"(st + A_BYTES + B_BYTES + S_BYTES + wave * 256), "v"(ws_src + 2 * kt) : "memory");
+            lds_load_x4(st + A_BYTES + wave * 2048 + b * 1024, b_src[b] + 64 * kt);
+        lds_load_dword(st + A_BYTES + B_BYTES + wave * 256, xs_src + 4 * kt);
+        lds_load_ushort(st + A_BYTES + B_BYTES + S_BYTES + wave * 256, ws_src + 2 * kt);
     };
     typedef const __attribute__((address_space(3))) i32x4* l_i32x4;
     typedef const __attribute__((address_space(3))) u32x4* l_u32x4;

@@ -160,3 +160,18 @@ def test_gemm_plan_policy():
         qe_amd.set_tuning("gemm_tile", 0)
         qe_amd.set_tuning("gemm_slices", 0)
         qe_amd.set_tuning("gemm_split_k", 1)
+
+
+def test_inline_assembly_names_what_it_writes():
+    """Every asm statement that sets m0 (the LDS address of a load into LDS) lists
+    it as clobbered, so the compiler keeps nothing there across it."""
+    import glob
+    seen = 0
+    for path in glob.glob(os.path.join(ROOT, "qwen-engine_amd", "csrc", "*.[hc]*")):
+        with open(path) as f:
+            statements = re.findall(r"\basm\s+volatile\s*\((.*?)\);", f.read(), re.S)
+        for text in statements:
+            if re.search(r"\bm0\s*,", text):
+                seen += 1
+                assert '"m0"' in text.rsplit(":", 1)[1], (path, text)
+    assert seen == 4
