@@ -443,8 +443,10 @@ __global__ __launch_bounds__(128) void flash_decode_stage2_kernel(const float* _
 // multiply-add), fp32 accumulation.  The reference value a row subtracts is
 // its running max, renewed only when the max has grown by more than
 // kPrefillLag (the probabilities then reach at most 2^kPrefillLag, and their
-// relative precision in fp16 does not change); each row decides for itself,
-// so its bits do not depend on the rows beside it.
+// relative precision in fp16 does not change).  Each row decides for itself:
+// unsplit and with one key group its bits do not depend on the rows beside it.
+// The key splits and the two key groups, which follow from the whole launch
+// (rows, context, workspace), change the order of its sums.
 constexpr int kPaRows = 128;     // rows per block
 constexpr int kPaKeys = 64;      // keys per tile
 constexpr int kPaTileBytes = kPaKeys * kHeadDim * 2;
@@ -502,7 +504,7 @@ __global__ __launch_bounds__(256 * KG, 2) void prefill_attention_kernel(PrefillA
     const int rows = p.T * p.group;
     const int base = p.ctl != nullptr ? p.ctl->seq_pos : 0;
     const int nt_all = prefill_tiles(rb, rows, p.group, base, p.max_seq);
-    const int live = prefill_live_splits(nt_all, p.splits);
+    const int live = KG == 2 ? 1 : prefill_live_splits(nt_all, p.splits);  // two groups: never split (the launcher)
     if (split >= live) return;
     const int it0 = static_cast<int>((static_cast<long long>(split) * nt_all) / live);
     const int it1 = static_cast<int>((static_cast<long long>(split + 1) * nt_all) / live);
@@ -512,10 +514,9 @@ __global__ __launch_bounds__(256 * KG, 2) void prefill_attention_kernel(PrefillA
     const int run_end = it1 * kPaKeys - 1;  // last key of the run
     const int lim = min(min(base + qi, p.max_seq - 1), run_end);  // last key this row takes here
     // keys every row of the wave takes: tiles that end at or before it skip the mask
-    const int wave_lim = min(min(base + min(rb * kPaRows + wave * 32, rows - 1) / p.group, p.max_seq - 1), run_end);
+    const int wave_lim = __builtin_amdgcn_readlane(lim, 0);
     // the last key that any row of the wave takes here
-    const int wave_last =
-        min(min(base + min(rb * kPaRows + wave * 32 + 31, rows - 1) / p.group, p.max_seq - 1), run_end);
+    const int wave_last = __builtin_amdgcn_readlane(lim, 31);
     const int key_max = max(0, min(base + p.T, p.max_seq) - 1);  // the last key that holds anything
     constexpr float kScale = 1.4426950408889634f * 0.08838834764831845f;  // log2(e) / sqrt(128)
 
@@ -760,7 +761,6 @@ __global__ __launch_bounds__(256 * KG, 2) void prefill_attention_kernel(PrefillA
         const float m = fmaxf(mref, mo);
         const float wm = mref == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mref - m);
         const float wo = mo == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mo - m);
-        mref = m;
         // one order for both groups, so that both hold the same sum
         const float l0 = kg == 0 ? lsum * wm : lo * wo, l1 = kg == 0 ? lo * wo : lsum * wm;
         lsum = l0 + l1;
@@ -774,7 +774,7 @@ __global__ __launch_bounds__(256 * KG, 2) void prefill_attention_kernel(PrefillA
     }
     if (r >= rows) return;
     constexpr int ND = KG == 2 ? 2 : 4;  // 32-dim tiles this wave writes, from dim 64 kg
-    if (live == 1) {
+    if (KG == 2 || live == 1) {
         const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
         uint16_t* o = p.out + static_cast<size_t>(qi) * p.out_stride + qh * kHeadDim + 64 * kg;
 #pragma unroll
@@ -790,10 +790,10 @@ __global__ __launch_bounds__(256 * KG, 2) void prefill_attention_kernel(PrefillA
         return;
     }
     const size_t prow = (static_cast<size_t>(split) * p.nkv + kvh) * rows + r;
-    if (h == 0 && kg == 0) *reinterpret_cast<float2*>(p.part_ml + 2 * prow) = make_float2(mref, lsum);
-    float* po = p.part_o + prow * kHeadDim + 64 * kg;
+    if (h == 0) *reinterpret_cast<float2*>(p.part_ml + 2 * prow) = make_float2(mref, lsum);
+    float* po = p.part_o + prow * kHeadDim;
 #pragma unroll
-    for (int dt = 0; dt < ND; ++dt)
+    for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
             *reinterpret_cast<float4*>(po + 32 * dt + 8 * g + 4 * h) =
@@ -1016,11 +1016,11 @@ int launch_prefill_attention(const uint16_t* q, const uint16_t* layer_k_cache, c
     // block per CU: blocks half as long leave a smaller last round (4096 rows
     // from position 0, 384 blocks: 75 against 88 us).  With fewer blocks a
     // wave that has its SIMD to itself finishes its tiles sooner (509 rows: 13.7
-    // against 16.3 us).
+    // against 16.3 us).  More blocks than CUs also leave no room for splits (above).
     if (!aligned(layer_k_cache, 16) || !aligned(layer_v_cache, 16))
         prefill_attention_kernel<1, false><<<static_cast<unsigned>(blocks * p.splits), 256, 0, stream>>>(p);
     else if (blocks > cus)
-        prefill_attention_kernel<2, true><<<static_cast<unsigned>(blocks * p.splits), 512, 0, stream>>>(p);
+        prefill_attention_kernel<2, true><<<static_cast<unsigned>(blocks), 512, 0, stream>>>(p);
     else
         prefill_attention_kernel<1, true><<<static_cast<unsigned>(blocks * p.splits), 256, 0, stream>>>(p);
     if (p.splits > 1)

@@ -385,6 +385,39 @@ def test_prefill_attention_infinity_at_a_later_position(qe, T, base, nq, nkv, ma
         qe.gemm_release_workspace(s)
 
 
+@pytest.mark.parametrize("T,chunk,nq,nkv,max_seq,same", [
+    (960, 123, 12, 2, 1000, True), (960, 320, 8, 8, 1000, True),  # below 1024 positions: neither splits nor key groups
+    (1500, 500, 12, 2, 2048, False), (1500, 400, 32, 32, 2048, False)])
+def test_prefill_attention_in_chunks(qe, T, chunk, nq, nkv, max_seq, same):
+    """Rows attended in one launch and in chunks of it, on a stream with a
+    workspace.  Without splits and key groups a row's bits do not depend on the
+    launch; else its sums have another order, and both results lie within the
+    bound of test_prefill_attention_splits_and_groups of the exact one."""
+    D = 128
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T + chunk)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g).half()
+    q, kc, vc = rnd(T, nq * D), rnd(nkv, max_seq, D), rnd(nkv, max_seq, D)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    qe.gemm_reserve_workspace(s)
+
+    def run(step):
+        out = empty((T, nq * D), torch.float16)
+        torch.cuda.synchronize()
+        for r in range(0, T, step):
+            n = min(step, T - r)
+            qe.launch_attention_gqa_prefill(q[r:r + n], kc, vc, out[r:r + n], _ctl(r), n, stream=s, num_q_heads=nq,
+                                            num_kv_heads=nkv, head_dim=D, max_seq_len=max_seq, hidden_size=nq * D)
+            s.synchronize()
+        return out
+
+    whole, parts = run(T), run(chunk)
+    qe.gemm_release_workspace(s)
+    assert torch.equal(whole.view(torch.int16), parts.view(torch.int16)) == same
+    assert (whole.double() - parts.double()).abs().max().item() <= 2 * (4.5 * 2.0 ** -10 + 2.0 ** -11)
+
+
 def test_captured_prefill_attention_keeps_to_its_own_buffers(qe):
     """A graph of a prefill attention captured on a stream with a workspace is
     replayed on another stream after the workspace was given up: the former

@@ -90,6 +90,24 @@ def test_recorded_prefill_attention_takes_no_workspace(recorder):
     """)
 
 
+def test_two_key_groups_are_never_split(recorder):
+    """More blocks than CUs: two key groups a block, one kernel, whatever the
+    context and the workspace; with half as many one group, split in three (what
+    the workspace holds)."""
+    launch_recorder.run(recorder, """
+        reserve()
+        for rows, blocks in ((1370, 257), (3002, 563), (680, 128)):
+            for max_seq in (1024, 4096, 32768):
+                R.recorder_reset(0)
+                attention(0, rows, 24, 1, max_seq)
+                e = events()
+                if blocks > 256:
+                    assert len(e) == 1 and e[0].block == 512 and e[0].grid == (blocks, 1, 1), e
+                else:
+                    assert len(e) == 2 and e[0].block == 256 and e[0].grid == (3 * blocks, 1, 1), e
+    """)
+
+
 @pytest.mark.parametrize("tiled", [False, True])
 def test_forced_tile_takes_the_slices_of_its_own_family(recorder, tiled):
     """With gemm_tile 1..4 and no slice count forced, a launch runs what
