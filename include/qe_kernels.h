@@ -279,7 +279,9 @@ int qe_launch_sample_and_advance(const uint16_t* logits, float* sample_scratch_v
  * accumulation, fp16 out; residual added as fp16(fp16(acc) + res) like the
  * fp16 GEMM).  The int8 prefill alternative named in design_draft.md:117-120
  * of the reference; no counterpart in its API.  K % 128 == 0, 16-byte
- * aligned Q8_1 rows and weights. */
+ * aligned Q8_1 rows and weights.  input_sum8 must be given as for the other Q8_1
+ * consumers (not NULL, 16-byte aligned) but is not read: the weights enter as
+ * q - 8. */
 int qe_launch_gemm_prefill_w4a8(const uint32_t* qweight, const uint16_t* scales, const int8_t* input_q8,
                                 const float* input_scale, const int32_t* input_sum8, const uint16_t* residual,
                                 uint16_t* output_y, int M, int N, int K, hipStream_t stream);

@@ -1186,6 +1186,7 @@ extern "C" int qe_launch_gemm_prefill_dual_gate_up_swiglu_w4a16(const uint32_t* 
 
 // ---- W4A8 prefill GEMM entry points --------------------------------------------------
 namespace {
+// s8 is part of the Q8_1 format and required as such; the kernel takes the zero point out of the weights and never reads it
 int check_gemm_a8(const char* what, const int8_t* q8, const float* xs, const int32_t* s8, int M, int K) {
     QE_REQUIRE(q8 && xs && s8, "%s: Q8_1 input pointers must not be NULL", what);
     QE_REQUIRE(M >= 0, "%s: M=%d", what, M);
@@ -1210,7 +1211,6 @@ extern "C" int qe_launch_gemm_prefill_w4a8(const uint32_t* qweight, const uint16
     p.out_stride[0] = N;
     p.A8 = input_q8;
     p.A8_scale = input_scale;
-    p.A8_sum8 = input_sum8;
     p.residual = residual;
     p.M = M;
     p.N = N;
@@ -1247,7 +1247,6 @@ extern "C" int qe_launch_gemm_prefill_qkv_w4a8(const qe_qkv_view* view, const in
     p.col_begin[2] = q_dim + kv_dim;
     p.A8 = input_q8;
     p.A8_scale = input_scale;
-    p.A8_sum8 = input_sum8;
     p.M = M;
     p.N = q_dim + 2 * kv_dim;
     p.K = in_features;
@@ -1272,7 +1271,6 @@ extern "C" int qe_launch_gemm_prefill_dual_gate_up_swiglu_w4a8(const uint32_t* g
     p.out_stride[0] = intermediate_size;
     p.A8 = input_q8;
     p.A8_scale = input_scale;
-    p.A8_sum8 = input_sum8;
     p.M = M;
     p.N = 2 * intermediate_size;
     p.K = hidden_size;

@@ -16,7 +16,6 @@ struct GemmParams {
     const uint16_t* residual;
     const int8_t* A8;         // W4A8 variant: Q8_1 rows of the activation
     const float* A8_scale;
-    const int32_t* A8_sum8;
     float* ws;         // split-K partials (slices > 1 only)
     int M, N, K;       // N = virtual columns (SwiGLU: 2*I)
 };

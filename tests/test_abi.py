@@ -72,6 +72,16 @@ def test_null_pointers_rejected_on_host():
     assert "NULL" in L.qe_last_error().decode()
 
 
+def test_w4a8_gemm_still_requires_the_sums_on_host():
+    """The W4A8 prefill GEMM does not read input_sum8, but a Q8_1 input without
+    it, or with it misaligned, is refused as by the other Q8_1 consumers."""
+    import qe_amd
+    L = qe_amd.lib()
+    for s8, why in ((None, "NULL"), (0x1000 + 4, "aligned")):
+        assert L.qe_launch_gemm_prefill_w4a8(0x1000, 0x1000, 0x1000, 0x1000, s8, None, 0x1000, 4, 128, 128, None) == 1
+        assert why in L.qe_last_error().decode()
+
+
 def test_engine_rejects_bad_config_on_host():
     import ctypes
     import qe_amd

@@ -231,6 +231,16 @@ def test_gemm_w4a8_rows_equal_w4a8_gemv(qe, orc, M, N, K):
     assert_fp16_close(host(out)[rows], ex, bd, ref, what=f"gemm_w4a8 {M}x{N}x{K}")
 
 
+def test_gemm_w4a8_does_not_read_the_sums(qe, orc):
+    M, N, K = 70, 130, 384
+    qw, sc = orc.synth_w4(31, N, K)
+    q8, xs, s8 = _q8_rows(qe, _A(orc, M, K, 19))
+    out = [empty((M, N), torch.float16) for _ in range(2)]
+    for o, s in zip(out, (s8, torch.full_like(s8, 0x55555555))):
+        qe.launch_gemm_prefill_w4a8(dev(qw), dev(sc), q8, xs, s, None, o, M, N, K)
+    assert np.array_equal(host(out[0]).view(np.uint16), host(out[1]).view(np.uint16))
+
+
 def test_gemm_w4a8_residual_qkv_swiglu(qe, orc):
     M, H, I = 96, 1536, 512
     A = _A(orc, M, H, 16)
