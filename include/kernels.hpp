@@ -7,8 +7,9 @@
 //
 // Every launcher of kernels.cuh that src/engine.cu calls is declared here:
 // the matrix path, and the embedding, RoPE/KV-append, attention and sampling
-// launchers of the decode and prefill loops.  The prefill GEMMs that split K
-// keep their partial sums in a workspace per stream (see qe_kernels.h).
+// launchers of the decode and prefill loops.  Prefill GEMMs that split K and
+// prefill attention that splits the keys keep their partial sums in a workspace
+// per stream, registered ahead of time (see qe_kernels.h).
 #pragma once
 
 #include <hip/hip_fp16.h>

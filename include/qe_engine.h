@@ -6,8 +6,8 @@
  * (include/qwenbin.h).  One engine = one HIP stream, one device arena
  * (allocated at create), one captured decode graph.  Besides the weights
  * (or the .qwenbin payload, one device copy), the KV cache and the
- * activations, the arena holds a 32 MiB split-K workspace for the prefill
- * GEMMs (registered for the engine's stream) and, unless
+ * activations, the arena holds a 32 MiB split workspace for the prefill
+ * GEMMs and prefill attention (registered for the engine's stream) and, unless
  * qe_set_tuning("engine_tiled_prefill", 0) was set before create, a tiled
  * copy of every layer matrix for the prefill GEMMs (+0.75 GB at
  * Qwen2.5-1.5B: about 0.8x the layer weights).  The switch is read once at

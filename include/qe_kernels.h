@@ -14,15 +14,25 @@
  * under HIP graph capture.  `residual` may alias the output.  A NULL
  * optional pointer means "skip", as in the reference.  No launcher
  * allocates (the reference's launchers keep no state and allocate nothing,
- * src/kernels/gemm_prefill.cu:616-684).  The prefill GEMMs may split K over
- * several blocks and then keep fp32 partial sums in a workspace registered
- * for the launching stream, ahead of time, by qe_gemm_reserve_workspace (the
- * library allocates 32 MiB) or qe_gemm_attach_workspace (caller memory).  A
- * stream without a workspace runs its GEMMs without K slices, eagerly and
- * under graph capture alike: the plan, and so the bits, of a launch depend
- * only on the shape, the qe_set_tuning switches and whether the stream holds
- * a workspace.  GEMMs on different streams never share partials.
- * hipStreamPerThread never holds a workspace (it names a different stream
+ * src/kernels/gemm_prefill.cu:616-684).
+ *
+ * The split workspace.  The prefill GEMMs may split K, and prefill attention
+ * the keys, over several blocks; they then keep fp32 partial sums in a workspace
+ * registered for the launching stream, ahead of time, by
+ * qe_gemm_reserve_workspace (the library allocates 32 MiB) or
+ * qe_gemm_attach_workspace (caller memory).  A stream without a workspace runs
+ * both unsplit.  The plan, and so the bits, of a launch depend only on the
+ * shape (attention: max_seq_len too, and in the engine the context length), the
+ * qe_set_tuning switches, whether the stream holds a workspace and how large,
+ * the alignment of tiled scales (4 bytes or not) and of the KV caches (16 bytes
+ * or not), and for attention on whether the launch is being recorded.
+ *   Threads: launches on different streams never share partials, and launches
+ * of several threads on one stream are enqueued whole, one after the other.
+ *   Graphs: a split GEMM recorded into a graph keeps the workspace's address.
+ * Replay such a graph while that workspace stays registered, and on its stream
+ * or with no split launch in flight there.  Prefill attention recorded into a
+ * graph runs unsplit and touches no workspace.
+ *   hipStreamPerThread never holds a workspace (it names a different stream
  * in every thread); the null stream is the device's legacy stream.
  *
  * Return value: QE_OK, or a QE_ERR_* code; qe_last_error() then describes
@@ -141,28 +151,30 @@ int qe_launch_rmsnorm_gemv_dual_gate_up_swiglu_w4a16(const uint16_t* input, cons
 
 /* ---- prefill dequant-GEMM (MFMA) ----------------------------------------- */
 
-/* Allocates a 32 MiB split-K workspace for `stream` on the current device
+/* Allocates a 32 MiB split workspace for `stream` on the current device
  * (hipMalloc; the only allocation of the kernel API) and registers it, so
- * prefill GEMMs on that stream may split K.  Call it before the first GEMM
- * on the stream, outside graph capture (QE_ERR_INVALID_ARGUMENT while the
+ * prefill GEMMs on that stream may split K and prefill attention the keys.
+ * Call it before the first of them on the stream, outside graph capture (QE_ERR_INVALID_ARGUMENT while the
  * stream is capturing, or for hipStreamPerThread).  At most 64 streams per
  * device hold a workspace (QE_ERR_UNSUPPORTED beyond).  No counterpart in the
  * reference (its GEMMs never split K). */
 int qe_gemm_reserve_workspace(hipStream_t stream);
 
 /* Registers caller memory (>= 1 MiB, 256-byte aligned; at most 32 MiB is
- * used) as the split-K workspace of `stream` on the current device, in place
+ * used) as the split workspace of `stream` on the current device, in place
  * of one allocated by qe_gemm_reserve_workspace (which is then freed).  The
  * memory must stay valid until qe_gemm_release_workspace(stream).  No
  * counterpart in the reference. */
 int qe_gemm_attach_workspace(hipStream_t stream, void* workspace, size_t bytes);
 
 /* Drops the workspace of `stream` on the current device (freed if the
- * library allocated it; call it before destroying the stream).  Later GEMMs
- * on the stream run without K slices.  QE_OK also when there was none. */
+ * library allocated it; call it before destroying the stream, and not while a
+ * graph that holds a split GEMM of the stream may still be replayed).  Later
+ * GEMMs and prefill attention on the stream run unsplit.  QE_OK also when there
+ * was none. */
 int qe_gemm_release_workspace(hipStream_t stream);
 
-/* Number of hipMalloc calls the library has made for GEMM workspaces in this
+/* Number of hipMalloc calls the library has made for split workspaces in this
  * process (only qe_gemm_reserve_workspace makes them).  Test hook. */
 long qe_gemm_workspace_allocations(void);
 
@@ -402,7 +414,13 @@ int qe_launch_attention_combine_gemv_o_w4a8(const float* splitk_partial_out, con
                                             const qe_device_control_block* d_control, int out_features,
                                             int num_q_heads, int head_dim, int max_seq_len, hipStream_t stream);
 
-/* Replaces launch_attention_gqa_prefill, include/kernels.cuh:195-207. */
+/* Replaces launch_attention_gqa_prefill, include/kernels.cuh:195-207.  With
+ * max_seq_len >= 1024 on a stream with a split workspace the keys of a launch
+ * with few rows are split over blocks (a second kernel merges the splits); with
+ * more blocks of 128 (query, head) rows than CUs a block's keys are shared by two
+ * groups of waves.  Both follow from the whole launch, so the rows of a launch and
+ * of its chunks may differ by the order of fp32 sums; otherwise they are equal
+ * bit for bit. */
 int qe_launch_attention_gqa_prefill(const uint16_t* q, const uint16_t* layer_k_cache, const uint16_t* layer_v_cache,
                                     uint16_t* attn_out, const qe_device_control_block* d_control, int num_tokens,
                                     hipStream_t stream, int num_q_heads, int num_kv_heads, int head_dim,
@@ -417,8 +435,8 @@ int qe_launch_attention_gqa_prefill(const uint16_t* q, const uint16_t* layer_k_c
 int qe_stream_read(const void* data, size_t bytes, uint32_t* sink, hipStream_t stream);
 
 /* Process-wide tuning switches (no counterpart in the reference):
- *   "gemm_split_k" 0/1 (default 1) - split K across blocks for prefill GEMMs
- *   whose tile grid leaves CUs idle;
+ *   "gemm_split_k" 0/1 (default 1) - use split workspaces: K of prefill GEMMs
+ *   whose tile grid leaves CUs idle, and the keys of prefill attention;
  *   "gemm_tile" 0..8 (default 0 = chosen per shape) - force the prefill GEMM
  *   block tile: 1 64x64, 2 64x128, 3 128x64, 4 128x128 (rows x columns); tiled
  *   weights only (ignored for others): 5 128x256, 6 128x256 and 7 128x128 with
