@@ -564,6 +564,27 @@ float predict_dma_us(const DmaCost& t, int M, int N, int K, int slices, int cus)
     return us;
 }
 
+// Where an automatic plan may name an LDS-ring kernel at all.  The model above
+// was fitted on weights that stay in the caches and at one model's widths.  With
+// weights from memory (600 MB rotated, as a whole model does), hidden 1024..2048,
+// intermediate 2048..8960 and M = 72..1400 (and to 4096 at Qwen2.5-1.5B's widths), the
+// register-staged plan's time over the ring kernel's was (launches measured):
+//   128x256, one group: up to 1.5 blocks per CU 0.97..1.00 (8), above it
+//   0.97..1.19 (23);
+//   two groups, more than one round of a block per CU: 0.79..0.93 (4);
+//   128x256, two groups, within a round: under 3/4 of the CUs 0.94..1.05 (13),
+//   from there 0.99..1.24 (24), but split with under 16 steps a group 0.88 (2);
+//   128x128, two groups, within a round: split 0.84..1.02 (8), K above 2048
+//   0.98..1.00 (4), else under 1280 rows 0.91..1.02 (41), from there 0.98..1.10 (10).
+bool dma_worth(int i, int M, int N, int K, int slices, int cus) {
+    const DmaCost& t = kDma[i];
+    const long long blocks = static_cast<long long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * slices;
+    if (t.groups == 1) return 2 * blocks > 3LL * cus;
+    if (blocks > cus) return false;
+    if (t.bn == 256) return 4 * blocks >= 3LL * cus && (slices == 1 || K >= 2048 * slices);
+    return slices == 1 && M >= 1280 && K <= 2048;
+}
+
 // Time of the kernel for a few rows (gemm_skinny.hip): launch and one load
 // latency, the bytes a block takes from L2 (weights of the .qwenbin layout cost
 // half again, in 64-byte pieces) at 45 GB/s per CU, the weights at 5 TB/s.
@@ -580,10 +601,10 @@ float predict_skinny_us(int M, int N, int K, bool tiled, int cus) {
 // predicts fastest among those whose split-K partials fit ws_floats, under the
 // gemm_tile / gemm_slices overrides.  ti: 0..3 the register-staged tiles, 4..6
 // the kernels of gemm_dma.hip (tiled weights only).  Those win where a launch
-// has enough steps to fill (gate/up at M = 1024 72 against 78 us, 2048 120
-// against 136, 4096 215 against 265; down at M = 2048 70 against 80; QKV at M =
-// 2048 19.6 against 25) and lose 1 to 6 us on shorter ones (QKV at M = 512 15.7
-// against 10.0).  The register-staged model is 10 % low around the crossing and
+// has enough steps to fill (gate/up at M = 1024 71 against 75 us, 2048 119
+// against 131, 4096 223 against 261; down at M = 2048 71 against 76; QKV at M =
+// 2048 20.6 against 22.6) and lose elsewhere (gate/up at M = 128 19.1 against 17.7;
+// dma_worth has the sides).  The register-staged model is 10 % low around the crossing and
 // 15 to 25 % low past M = 1280, hence the factors.
 // A forced tile takes the slice count of the best plan of its own family
 // (register-staged, LDS ring); only a launch with no tile forced is free to
@@ -604,22 +625,22 @@ void plan_gemm(int M, int N, int K, size_t ws_floats, bool tiled, int& ti, int& 
     auto fits = [&](int i, int s) {
         return i < 4 ? fits_tile(kTiles[i].bm, kTiles[i].bn, s) : fits_tile(kDma[i - 4].bm, kDma[i - 4].bn, s);
     };
+    const int f = gemm_forced_tile() - 1, n = gemm_forced_slices();
+    const bool force_staged = f >= 0 && f < 4, force_dma = f >= 4 && f < 4 + kDmaTiles && tiled && ring;
+    const bool force_few = f == kSkinnyTile && M <= kSkinnyRows;
+    const bool any = !force_staged && !force_dma && !force_few && !staged_only && !gemm_staged_only();
     float best = 1e30f;
     auto search = [&](int first, int last) {
         for (int i = first; i < last; ++i) {
             for (int s : {1, 2, 3, 4, 6}) {
                 if (s > 1 && !gemm_split_k_enabled()) break;
-                if (!fits(i, s)) continue;
+                if (!fits(i, s) || (!force_dma && i >= 4 && !dma_worth(i - 4, M, N, K, s, cus))) continue;
                 const float us = i < 4 ? predict_us(tiled ? kTilesTiled[i] : kTiles[i], M, N, K, s, cus)
                                        : predict_dma_us(kDma[i - 4], M, N, K, s, cus);
                 if (us < best) { best = us; ti = i; slices = s; }
             }
         }
     };
-    const int f = gemm_forced_tile() - 1, n = gemm_forced_slices();
-    const bool force_staged = f >= 0 && f < 4, force_dma = f >= 4 && f < 4 + kDmaTiles && tiled && ring;
-    const bool force_few = f == kSkinnyTile && M <= kSkinnyRows;
-    const bool any = !force_staged && !force_dma && !force_few && !staged_only && !gemm_staged_only();
     ti = 0;
     slices = 1;
     if (!force_dma) search(0, 4);

@@ -177,6 +177,33 @@ def test_launch_plan_names_the_kernel_that_runs(recorder, tiled, setting):
     """)
 
 
+def test_automatic_plans_leave_the_ring_where_it_is_slower(recorder):
+    """Sides of the rule that admits an LDS-ring kernel to an automatic plan; a
+    forced tile is not asked."""
+    launch_recorder.run(recorder, """
+        reserve()
+        def kernel(M, N, K):
+            t, s = I(), I()
+            ok(L.qe_gemm_prefill_launch_plan(I(M), I(N), I(K), I(1), ctypes.byref(t), ctypes.byref(s)))
+            R.recorder_reset(0)
+            gemm(M, N, K, 0, True)
+            assert ("_dma_" in events()[0].kernel) == (t.value in (5, 6, 7)), (M, N, K, t.value)
+            return t.value
+        for M, N, K, ring in ((72, 17920, 2048, 0), (128, 17920, 1536, 0), (256, 17920, 1536, 0),  # too few blocks
+                              (384, 17920, 1536, 6), (700, 17920, 1536, 5), (1024, 17920, 1536, 5), (4096, 17920, 1536, 5),
+                              (850, 12288, 1536, 0), (1200, 12288, 1536, 5),  # up to 1.5 blocks a CU, above it
+                              (512, 17920, 2048, 0), (700, 12288, 2048, 0),   # more than a round of two-group blocks
+                              (512, 1536, 4096, 0), (700, 1024, 4096, 0),     # 128x128 split
+                              (1200, 2048, 4096, 0), (1400, 1536, 6144, 6),   # 128x256 split, short and long
+                              (1200, 2048, 1536, 0), (2048, 2048, 1536, 7)):  # 128x128, rows
+            got = kernel(M, N, K)
+            assert got == ring if ring else got <= 4, (M, N, K, got, ring)
+        for tile in (5, 6, 7):
+            tune("gemm_tile", tile)
+            assert kernel(128, 17920, 1536) == tile
+    """)
+
+
 @pytest.mark.parametrize("tile", [0, 5, 6, 7])
 def test_tiled_scales_at_an_odd_half_take_the_staged_kernels(recorder, tile):
     """Tiled scales need 2-byte alignment only. The LDS-ring kernels fetch them in
