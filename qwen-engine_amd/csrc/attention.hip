@@ -332,12 +332,24 @@ __global__ __launch_bounds__(NT) void flash_decode_stage1_kernel(const uint16_t*
     // (split, kv head) takes blocks with b % 8 = u % 8.  With heads in launch
     // order every XCD fetched every row: 3.43 -> 2.69 us at 128 positions, 7.1
     // -> 4.4 at 3000, 19.4 -> 10.4 at 16000 (12 q heads, 2 kv heads).
+    // With one q head per kv head there is nothing to share, and heads in launch
+    // order are the faster ones (28 caches in turn): 16 heads 7.35 -> 6.40 us at 2000
+    // positions, 4.25 -> 4.04 at 300; 8 heads 5.26 -> 4.94 and 3.38 -> 3.23.
     static_assert(kSplits % 8 == 0, "units fill the XCDs evenly");
     const int heads = group / GH;  // blocks per unit
-    const int x = blockIdx.x & 7, sl = blockIdx.x >> 3;
-    const int unit = x + 8 * (sl / heads);
-    const int split = unit % kSplits, kvh = unit / kSplits;
-    const int qh0 = kvh * group + (sl % heads) * GH;
+    int split, kvh, qh0;
+    if constexpr (SHARED) {
+        const int x = blockIdx.x & 7, sl = blockIdx.x >> 3;
+        const int unit = x + 8 * (sl / heads);
+        split = unit % kSplits;
+        kvh = unit / kSplits;
+        qh0 = kvh * group + (sl % heads) * GH;
+    } else {  // nothing to share: heads in launch order
+        const int nkv = gridDim.x / kSplits;
+        kvh = blockIdx.x % nkv;
+        split = blockIdx.x / nkv;
+        qh0 = kvh;
+    }
     const int gid = threadIdx.x >> 4, j = threadIdx.x & 15;
     // q and the split's first 64 rows are requested before the position is
     // known: with splits of 64 positions (contexts up to 16 * 64) the rows are

@@ -122,6 +122,12 @@ def test_flash_decode_attention(qe, orc, nq, nkv, seq_pos):
     assert np.array_equal(host(s8), -8 * host(q8).astype(np.int32).reshape(-1, 8).sum(1))
 
 
+@pytest.mark.parametrize("heads,seq_pos", [(1, 100), (3, 1500), (8, 0), (8, 2000), (16, 1023)])
+def test_flash_decode_one_q_head_per_kv_head(qe, orc, heads, seq_pos):
+    """No rows to share between blocks: heads run in launch order."""
+    test_flash_decode_attention(qe, orc, heads, heads, seq_pos)
+
+
 @pytest.mark.parametrize("nq,nkv,seq_pos,res", [(12, 2, 0, True), (12, 2, 300, True), (12, 2, 4095, False),
                                                  (16, 2, 77, True), (8, 1, 1000, False), (4, 4, 17, True),
                                                  (12, 2, 63, False), (12, 2, 64, True), (12, 2, 1500, True)])
