@@ -699,19 +699,21 @@ int launch_gemm(GemmParams p, hipStream_t stream, const char* what, Workspace ws
 // ---- W4A8 variant: int8 activations on the int8 matrix cores (gemm_w4a8.hip) --------
 // Rows per block and K slices, from a sweep over M in {8..1500} at the
 // Qwen2.5-1.5B shapes and gate/up at hidden 1024..2048, weights from memory.  128
-// rows where such tiles fill most of one round of two blocks per CU (8192 x 1024 at
-// M = 850, 448 tiles: 22.8 us against 27.0 with 64 rows) or more than one by an
-// eighth (17920 x 1536 at M = 850, 980 tiles: 55.0 against 63.7; at 400 and 512, 560
-// tiles: 39.0 against 34.7 and 43.2 against 42.8), or where few tiles have a long K
-// (down at M = 512 24.5 against 25.7, at 1024 37 against 42; at 300 20.5 against 20.1).  Slices: one block per CU where that fills
-// the chip (down at M = 300 4 slices 20.1 us, 8 21.0); else two per CU if a slice
-// keeps 12 groups (down at M = 1024 5 slices 37 us, 2 42; O at M = 1024 2 slices
-// 15.7, unsplit 11.9).  A slice has at least 3 groups, a sum at most 16 slices.
+// rows where such tiles fill 7/8 of one round of two blocks per CU (8192 x 1024 at
+// M = 850, 448 tiles: 22.8 us against 27.0 with 64 rows; 17920 x 1536 at M = 300, 420
+// tiles: 29.2 against 28.6) or more than one by an eighth (17920 x 1536 at M =
+// 850, 980 tiles: 55.0 against 63.7; at 400 and 512, 560 tiles: 39.0 against 34.7
+// and 43.2 against 42.8), or where few tiles have a long K (down at M = 512 24.5
+// against 25.7, at 1024 37 against 42; at 300 20.5 against 20.1).  Slices: one block
+// per CU where that fills the chip (down at M = 300 4 slices 20.1 us, 8 21.0); else
+// two per CU if a slice keeps 12 groups (down at M = 1024 5 slices 37 us, 2 42; O at
+// M = 1024 2 slices 15.7, unsplit 11.9).  A slice has at least 3 groups, a sum at
+// most 16 slices.
 void plan_w4a8(int M, int N, int K, size_t ws_floats, int& bm, int& slices) {
     const int cus = cu_count(), G = K / 128;
     const auto tiles_of = [&](int rows) { return static_cast<long long>((N + 127) / 128) * ((M + rows - 1) / rows); };
     const long long t128 = tiles_of(128);
-    const bool one_round = t128 <= 2 * cus && 4 * t128 >= 5 * cus;
+    const bool one_round = t128 <= 2 * cus && 4 * t128 >= 7 * cus;
     bm = one_round || 4 * t128 >= 9 * cus || (t128 <= cus && t128 * G >= 12 * cus) ? 128 : 64;
     const long long tiles = tiles_of(bm);
     slices = 1;

@@ -205,13 +205,14 @@ def test_automatic_plans_leave_the_ring_where_it_is_slower(recorder):
 
 
 def test_w4a8_rows_per_block(recorder):
-    """Sides of the W4A8 tile rule: 128 rows a block where 128-row tiles fill 5/8 to
+    """Sides of the W4A8 tile rule: 128 rows a block where 128-row tiles fill 7/8 to
     all of a round, or from 9/8 of one on, or few tiles have a long K."""
     launch_recorder.run(recorder, """
         reserve()
-        for M, N, K, rows in ((300, 8192, 1024, 64), (600, 8192, 1024, 128), (1024, 8192, 1024, 128), (512, 17920, 1536, 64),
-                              (640, 14336, 1536, 64), (600, 17920, 1536, 128), (1500, 17920, 1536, 128),
-                              (300, 1536, 8960, 64), (1024, 1536, 8960, 128)):
+        for M, N, K, rows in ((300, 17920, 1536, 64), (700, 8192, 1024, 64), (850, 8192, 1024, 128),
+                              (1024, 8192, 1024, 128), (512, 17920, 1536, 64), (640, 14336, 1536, 64),
+                              (600, 17920, 1536, 128), (1500, 17920, 1536, 128), (300, 1536, 8960, 64),
+                              (1024, 1536, 8960, 128)):
             R.recorder_reset(0)
             gemm_w4a8(M, N, K)
             e = events()[0]
