@@ -446,11 +446,12 @@ __global__ __launch_bounds__(128) void flash_decode_stage2_kernel(const float* _
 // stored at c ^ swz(key): the 16-byte reads of K (16 keys, one chunk) and the
 // transposing reads of V (4 keys x 4 chunks a half wave) then touch every
 // bank once (0 conflicts counted).
-// Bound by the matrix cores and, beside them, the exponentials: at 1024 rows
-// on 15000 positions (12 q heads, 2 kv heads) 124 us = 790 TFLOP/s, of which the
-// MFMAs alone take 86 us.  Before, every wave read K for itself from L2 and no
-// keys were split: 450 us.  509 rows from position 0 23.2 -> 15.7 us, 4096 rows
-// 211 -> 74 us.
+// Bound by the matrix cores and, beside them, the exponentials: 1024 rows on
+// 15000 positions (12 q heads, 2 kv heads) take 113 us, and the merge of the
+// splits 7.5 (traced; together 0.81 PFLOP/s), with the MFMAs busy 54 % of the time
+// on a SIMD of a busy CU and 4.6 vector instructions an MFMA.  Before, every
+// wave read K for itself from L2 and no keys were split: 450 us.  509 rows from
+// position 0 23.2 -> 15.0 us, 4096 rows 211 -> 74 us.
 // Online softmax in the exp2 domain (1/sqrt(d) folded into the exponent's fused
 // multiply-add), fp32 accumulation.  The reference value a row subtracts is
 // its running max, renewed only when the max has grown by more than

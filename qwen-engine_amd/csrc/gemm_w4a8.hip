@@ -19,7 +19,9 @@
 // 128-group is one stage of a ring of D in LDS, filled by DMA (global_load_lds):
 // A rows of 128 bytes, 16-byte chunk ch stored at ch ^ (row / 2 % 8); weight
 // columns of 64 bytes, chunk c stored at c ^ (column / 4 % 4); the scales, a dword
-// a lane.  All operand reads then touch every bank once.
+// a lane.  The operand reads then touch every bank once; at 64 rows the x_scales of
+// rows 16 apart lie 256 bytes apart, in one bank, and a fragment's read of them takes
+// twice (0.5 conflict cycles an MFMA counted in all).
 //
 // What bounds it: the scaling, three vector instructions per result and group
 // against a quarter of an MFMA; and latency where a launch has few steps.  The
