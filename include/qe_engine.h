@@ -11,7 +11,9 @@
  * qe_set_tuning("engine_tiled_prefill", 0) was set before create, a tiled
  * copy of every layer matrix for the prefill GEMMs (+0.75 GB at
  * Qwen2.5-1.5B: about 0.8x the layer weights).  The switch is read once at
- * create.  qe_engine_arena_spans reports the arena's size.
+ * create.  qe_engine_arena_spans reports the arena's size.  Prefill in chunks
+ * of another size, and with qe_set_tuning("gemm_split_k", 0) (neither GEMMs nor
+ * attention split), may differ in the order of fp32 sums.
  *
  * Counterpart of the reference's QwenEngine (include/engine.cuh:104-226):
  * construction from a .qwenbin (load_model_file + setup_arena), prefill

@@ -104,7 +104,7 @@ struct qe_engine {
     int seq_pos = 0;
     bool tiled = false;        // prefill GEMMs read the tiled copies
     bool want_tiled = false;   // engine_tiled_prefill, read once at create
-    float* gemm_ws = nullptr;  // split-K workspace of the engine's stream (in the arena)
+    float* gemm_ws = nullptr;  // split workspace of the engine's stream (in the arena)
 
     std::vector<std::pair<size_t, size_t>> spans;  // (offset, bytes) of every buffer taken
     template <class T>
@@ -424,7 +424,7 @@ int q8_len(const qe_engine_config& c) {
     return std::max(c.intermediate_size, std::max(c.hidden_size, c.num_q_heads * c.head_dim));
 }
 
-// The engine's split-K workspace for its prefill GEMMs (registered for the
+// The engine's split workspace for its prefill GEMMs and attention (registered for the
 // engine's stream with qe_gemm_attach_workspace, released at destroy).
 constexpr size_t kEngineGemmWsBytes = size_t(32) << 20;
 

@@ -526,9 +526,9 @@ def stream_read(data, nbytes: int, sink, stream=None):
 
 
 def gemm_reserve_workspace(stream=None):
-    """qe_gemm_reserve_workspace: a 32 MiB split-K workspace for the stream
-    (the only allocation of the kernel API; prefill GEMMs on a stream
-    without one run without K slices)."""
+    """qe_gemm_reserve_workspace: a 32 MiB split workspace for the stream
+    (the only allocation of the kernel API; prefill GEMMs and prefill
+    attention on a stream without one run unsplit)."""
     _check(lib().qe_gemm_reserve_workspace(_stream(stream)), "qe_gemm_reserve_workspace")
 
 
@@ -542,7 +542,7 @@ def gemm_release_workspace(stream=None):
 
 
 def gemm_workspace_allocations() -> int:
-    """hipMalloc calls made so far for GEMM workspaces (test hook)."""
+    """hipMalloc calls made so far for split workspaces (test hook)."""
     return int(lib().qe_gemm_workspace_allocations())
 
 
@@ -564,5 +564,5 @@ def gemm_prefill_launch_plan(M, N, K, tiled=False):
 
 
 def set_tuning(key: str, value: int):
-    """qe_set_tuning: process-wide switches ("gemm_split_k")."""
+    """qe_set_tuning: process-wide switches ("gemm_split_k", "gemm_tile", ...)."""
     _call("qe_set_tuning", key.encode(), int(value))
